@@ -411,15 +411,11 @@ int gqk_plan(const gqk_shard* shards, int nshards, int64_t K, int M, int target_
     }
   } else {
     pi.form = GQK_FORM_GEMM;
-    // 64 / 128 tokens x 128 rows per tile up to 128 tokens (one decode of each weight); 256 x 256 above.
+    // Descriptor rows of two 64-row tiles up to 128 tokens, of four above; the launch picks its tile
+    // geometry (gqk_gemm_plan.hip).
     pi.bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;
-    // A layer with few 256-row groups keeps the 128 x 128 form up to 384 rows (768 for K up to
-    // 8192) when the 256 x 256 form would have fewer tiles than a quarter of the CUs (one
-    // workgroup each): its stream-K would leave most CUs idle and pad the last token block.
-    // Measured on the 5120- and 7168-row shards (20 / 28 groups of 256 rows): 13-30% faster at
-    // M = 129-384, 9-19% at 448-512 and (o_proj) 6-21% at 640-768 for K = 5120; qkv at 640-768
-    // (above the quarter) even to 11% slower, `down` (K = 17408) 5-19% slower at 448-512, and
-    // gate_up (136 groups) 6-22% slower at every M.
+    // A layer with few 256-row groups keeps the two-tile rows up to 384 tokens (768 for K up to 8192):
+    // 256 x 256 tiles would be fewer than a quarter of the CUs, and the launch never takes them there.
     if (pi.bm == 256 && (M <= 384 || (M <= 768 && nb <= 32))) {
       int64_t groups = 0;
       for (int i = 0; i < nshards; ++i) groups += ((shards[i].n + 63) / 64 + 3) / 4;

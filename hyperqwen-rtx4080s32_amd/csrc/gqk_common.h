@@ -132,7 +132,6 @@ GQK_LAYOUT(GQK_IQ4_XS, 136, 0, 128)
 // descriptor row of a grouped launch (int32 words)
 #define GQK_DESC_WORDS 16
 #define GQK_SPLIT_MAX 16   // split-K factor bound: the last workgroup loads every partial at once
-#define GQK_GEMM_MAX_WGS 1024   // persistent GEMM workgroups (up to three per CU) a launch may use
 // Arrival counters at the start of every workspace: one fixed region for every plan of every
 // layer (GEMV split tiles and GEMM stream-K tiles each index below it), so that one workspace per
 // device serves all layers and batch sizes: no plan's fp32 partials overlap another's counters.
@@ -171,4 +170,4 @@ void gqk_set_last_error(const char* msg);
 #define GQK_FORM_GEMV 1   // M <= 32, descriptor rows of (tile, k-range): M <= 16 the GEMV (in-register
                           // decode, MFMA per scale group, fp32 epilogue); 17..32 the mid form (g = 8:
                           // weights decoded to bf16 in registers, MFMA 32x32x16)
-#define GQK_FORM_GEMM 2   // M > 32: tile decoded to bf16 in LDS, MFMA 32x32x16
+#define GQK_FORM_GEMM 2   // M > 32: weights decoded to bf16 in registers, x staged in LDS, MFMA 32x32x16

@@ -16,7 +16,11 @@ REPO = os.path.dirname(ROOT)
 CSRC = os.path.join(ROOT, "csrc")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(PKG, "libgqk.so")
-SOURCES = ("gqk_api.hip", "gqk_codec.hip", "gqk_gemv.hip", "gqk_gemm.hip", "gqk_gguf.cpp")
+# (source, extra flags, object): the GEMM is compiled once per token-block count, side by side
+SOURCES = (("gqk_api.hip", (), "gqk_api.o"), ("gqk_codec.hip", (), "gqk_codec.o"), ("gqk_gemv.hip", (), "gqk_gemv.o"),
+           ("gqk_mid.hip", (), "gqk_mid.o"), ("gqk_gemm_plan.hip", (), "gqk_gemm_plan.o"),
+           *(("gqk_gemm.hip", (f"-DGQK_GEMM_MB={mb}",), f"gqk_gemm{mb}.o") for mb in (2, 4, 8)),
+           ("gqk_gguf.cpp", (), "gqk_gguf.o"))
 ARCH = os.environ.get("GQK_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -40,10 +44,10 @@ def build(jobs: int | None = None) -> str:
     os.makedirs(BUILD, exist_ok=True)
     objs = []
     cmds = []
-    for src in SOURCES:
-        obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+    for src, extra, name in SOURCES:
+        obj = os.path.join(BUILD, name)
         objs.append(obj)
-        cmds.append([HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
+        cmds.append([HIPCC, *FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
     with ThreadPoolExecutor(max_workers=jobs or min(len(cmds), os.cpu_count() or 4)) as ex:
         list(ex.map(_run, cmds))
     tmp = LIB + ".tmp"

@@ -35,8 +35,9 @@ UNQUANTIZED_TYPES = (0, 1, 30)
 # batch-row buckets of a grouped layer: the streaming plans serve M <= 4, 8, 16 (GEMV) and 17..32
 # (the mid form); GEMM above
 GEMV_BUCKETS = (4, 8, 16, 32)
-# GEMM plans: 64 x 128 tiles (33..64 rows), 128 x 128 (65..128), 129..384, 385..512 and 513..768
-# (256 x 256, or 128 x 128 for a layer with few 256-row groups), 256 x 256 above
+# GEMM plans: 33..64 rows, 65..128, 129..384, 385..512, 513..768 and above: descriptor rows of 128
+# weight rows up to 128 rows and for layers with few 256-row groups, of 256 otherwise (the launch
+# picks its tile geometry from the rows, the layer and the device)
 GEMM_PLAN_M = (64, 128, 384, 512, 768, 769)
 # From this many batch rows mul_mat_grouped takes the reference's dequant regime (its
 # gluon_mul_mat_tiles_grouped dequantizes the tiles and runs the vendor bf16 GEMM above 128 rows

@@ -32,7 +32,7 @@ extern "C" {
                            decode GEMV up to 16 rows (small shards up to 8 rows in its slab form,
                            plan bm = 2: a row per 32-row slab over the whole k-range), the mid form
                            (g = 8) for 17..32 (small shards at 9..32 rows in its slab form, bm = 2) */
-#define GQK_FORM_GEMM 2 /* M > 32: LDS-dequant bf16 MFMA GEMM (any M) */
+#define GQK_FORM_GEMM 2 /* M > 32: dequant bf16 MFMA GEMM, weights decoded in registers (any M) */
 
 #define GQK_CTR_BYTES 262144 /* the arrival-counter region at the start of every workspace */
 
@@ -54,7 +54,8 @@ typedef struct gqk_plan_info {
   int32_t m_max;      /* largest batch rows M the plan serves (GEMV: 4 * g) */
   int32_t g;          /* GEMV: groups of 4 tokens (1, 2, 4; 8 = the mid form, 17..32 rows, or its slab
                          form from 9 rows) */
-  int32_t bm;         /* GEMM: tokens per tile (64, 128, 256); GEMV (g <= 2): 1 when every wave streams
+  int32_t bm;         /* GEMM: the row-count class (64, 128, 256: two, two, four 64-row tiles per
+                         descriptor row; the launch picks its tile geometry from it); GEMV (g <= 2): 1 when every wave streams
                          exactly one 256-weight record (the launch takes the pipeline-free kernel),
                          2 for the slab form (a workgroup per 32-row half tile over the whole k-range,
                          one wave per pair of super-blocks, no split-K partials; with g = 8 the mid
@@ -114,7 +115,7 @@ int gqk_unrepack(const void* tiles, int ggml_type, int64_t n, int64_t K, void* W
  * runtime for the current device's count (initialising the runtime; 256 when no device is
  * visible).  target_wgs > 0 overrides the GEMV heuristic's target of resident waves (0 = eight per
  * CU), from which the waves per workgroup and the split-K factor follow.  GEMM plans (M > 32)
- * take their tile form from M and, at 129..384 rows (129..768 for K <= 8192), from the layer's
+ * take their descriptor rows from M and, at 129..384 rows (129..768 for K <= 8192), from the layer's
  * size against the CU count.  Replaces prepare_grouped_layer / descriptors / grouped_split_for
  * (gguf-plugin/gluon/tiles_grouped.py:237-299). */
 int gqk_plan(const gqk_shard* shards, int nshards, int64_t K, int M, int target_wgs, int cus, int32_t* desc,
@@ -158,7 +159,7 @@ int gqk_linear(const void* packed, const int32_t* desc_dev, const gqk_plan_info*
  * array of GQK_NOALLOC_SCRATCH_BYTES per GPU (held until the process ends; its address is taken
  * once per device on the first call, which also clears its counters with a fill kernel on
  * `stream`).  Allocates nothing.  A plan that needs more workspace at this M is refused with
- * GQK_ERR_SHAPE: GEMM plans above 64 rows on large layers, and GEMV plans whose split-K partials
+ * GQK_ERR_SHAPE: GEMM launches above 128 rows with many remainder tiles, and GEMV plans whose split-K partials
  * exceed the 32 MiB (those are 64 rows x m_max tokens x 4 bytes per partial slot: at most 4,096
  * slots at m_max = 32, 8,192 at 16, 32,768 at 4; e.g. a layer of 2,374 tiles at K = 16384 split 16
  * ways at M <= 4 needs ~39 MB).  Every call on one GPU shares that

@@ -1,0 +1,70 @@
+"""The GEMM's tile geometries at the sizes where they can go wrong: token and row remainders, row blocks
+past the last descriptor row, k-groups with unequal (or no) super-blocks, split and unsplit tiles,
+mixed types inside a workgroup, x rows further apart than 32-bit offsets reach.  Against the fp64
+product of the oracle's weights: rounding each weight and y once to bf16 moves an output by at most
+2^-9 (sum |x w| + |y|), fp32 accumulation by far less; over all outputs the error is under 1e-2."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ggml_ref as G
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(y, x, wf, bias=None):
+    x, wf, y = (np.asarray(v, np.float64) for v in (x, wf, y))
+    b = 0.0 if bias is None else np.asarray(bias, np.float64)[None]
+    ref, mag = x @ wf.T + b, np.abs(x) @ np.abs(wf).T
+    err = np.abs(y - ref)
+    return bool((err <= 2.0 ** -9 * (1.01 * mag + 1.01 * np.abs(ref)) + 1e-30).all()) and \
+        np.linalg.norm(err) <= 1e-2 * np.linalg.norm(ref)
+
+
+def _layer(dev, shards, K, seed):
+    import gguf_hip
+
+    rng = np.random.default_rng(seed)
+    raws = [G.make_weights(rng, n, K, wt) for wt, n in shards]
+    wf = np.concatenate([G.dequantize(r, wt) for r, (wt, _) in zip(raws, shards)])
+    return gguf_hip.pack_layer([torch.from_numpy(r).to(dev) for r in raws], [n for _, n in shards],
+                               [wt for wt, _ in shards]), wf
+
+
+@pytest.mark.parametrize("shards,nbk", [
+    ([(G.Q4_K, 1)], 1),                                     # one row, fewer super-blocks than k-groups
+    ([(G.Q3_K, 97)], 2),
+    ([(G.Q6_K, 161), (G.IQ3_S, 31)], 3),                    # a workgroup's waves on different types
+    ([(G.Q8_0, 330)], 5),
+    ([(G.IQ4_XS, 640), (G.Q2_K, 70), (G.Q5_0, 129)], 7),
+    ([(G.Q5_K, 2100)], 9),
+    ([(G.IQ4_NL, 33), (G.Q4_0, 64)], 13),
+])
+def test_geometries(dev, shards, nbk):
+    import gguf_hip
+
+    K = 256 * nbk
+    gl, wf = _layer(dev, shards, K, nbk)
+    bias = torch.randn(gl.n_total, device=dev).to(torch.bfloat16)
+    for M in (33, 63, 64, 65, 97, 128, 129, 255, 257):
+        print(shards, nbk, M, flush=True)
+        x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+        y = gguf_hip.mul_mat_grouped(x.to(dev), gl, bias)
+        assert _close(y.float().cpu().numpy(), x.float().numpy(), wf, bias.float().cpu().numpy()), M
+        for _ in range(2):
+            assert torch.equal(gguf_hip.mul_mat_grouped(x.to(dev), gl, bias), y), M
+    torch.cuda.synchronize()
+    assert int(gl.workspace[:65536].abs().sum()) == 0
+
+
+def test_rows_far_apart(dev):
+    """A row stride above 8 MiB: the rows go one by one."""
+    import gguf_hip
+
+    K, M, ldx = 512, 34, (1 << 22) + 64
+    gl, wf = _layer(dev, [(G.Q4_K, 130)], K, 3)
+    buf = torch.zeros((M - 1) * ldx + K, dtype=torch.bfloat16, device=dev)
+    x = buf.as_strided((M, K), (ldx, 1))
+    x.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16))
+    y = gguf_hip.mul_mat_grouped(x, gl)
+    assert _close(y.float().cpu().numpy(), x.float().cpu().numpy(), wf)
