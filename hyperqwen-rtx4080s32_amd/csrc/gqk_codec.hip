@@ -12,156 +12,167 @@
 
 namespace gqk {
 
-__device__ __forceinline__ float f16_at(const uint8_t* p) {
-  uint16_t b = (uint16_t)p[0] | ((uint16_t)p[1] << 8);
-  return (float)__builtin_bit_cast(_Float16, b);
+// Where a 256-weight record's bytes lie: RawSrc reads GGUF rows (any alignment), TileSrc a tile chunk in
+// LDS.  ld8<P>(j) / ld4 / ld2 / ld1: bytes j .. of plane P (j a multiple of the width; they never cross
+// a segment of the plane).
+template <int T, int P>
+__device__ __forceinline__ int raw_of(int j) {   // raw byte of byte j of plane P (equal segments concatenated)
+  constexpr gqk_plane pl = gqk_planes<T>::v.planes[P];
+  return pl.seg_off + (j / pl.seg_len) * pl.seg_stride + j % pl.seg_len;
 }
-
-__device__ __forceinline__ void scale_min_k4(const uint8_t* s, int j, int& sc, int& m) {
-  // gguf-plugin/gluon/kq_ref.py:17-27
-  if (j < 4) {
-    sc = s[j] & 63;
-    m = s[j + 4] & 63;
-  } else {
-    sc = (s[j + 4] & 0xF) | ((s[j - 4] >> 6) << 4);
-    m = (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
+template <int T, int P>
+__device__ __forceinline__ constexpr int plane_off() {
+  int o = 0;
+  for (int p = 0; p < P; ++p) o += gqk_planes<T>::v.planes[p].size;
+  return o;
+}
+template <typename V> __device__ __forceinline__ V load_any(const uint8_t* p) {
+  V v;
+  __builtin_memcpy(&v, p, sizeof v);
+  return v;
+}
+template <int T>
+struct RawSrc {
+  const uint8_t* rec;
+  static constexpr bool PACKED6 = false;
+  template <int P, typename V> __device__ __forceinline__ V ld(int j) const { return load_any<V>(rec + raw_of<T, P>(j)); }
+  template <typename V> __device__ __forceinline__ V raw(int b) const { return load_any<V>(rec + b); }
+};
+template <int T>
+struct TileSrc {
+  const uint8_t* chunk;   // plane-major chunk in LDS
+  int r;                  // row of the tile
+  static constexpr bool PACKED6 = true;
+  template <int P, typename V> __device__ __forceinline__ V ld(int j) const {
+    constexpr int W = gqk_col_width(gqk_planes<T>::v.planes[P].size), o = 64 * plane_off<T, P>();
+    return *(const V*)(chunk + o + ((j / W) * 64 + r) * W + j % W);
   }
+};
+
+__device__ __forceinline__ float f16_of(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
+template <int N>
+__device__ __forceinline__ float ub(const uint32_t (&v)[N / 4], int i) { return (float)((v[i >> 2] >> (8 * (i & 3))) & 0xFF); }
+__device__ __forceinline__ uint2 msk(const uint2& v, int sh, uint32_t m) { return make_uint2((v.x >> sh) & m, (v.y >> sh) & m); }
+__device__ __forceinline__ uint2 orr(const uint2& a, const uint2& b) { return make_uint2(a.x | b.x, a.y | b.y); }
+// bit i of byte b -> bit 4 of byte i (four at a time)
+__device__ __forceinline__ uint2 spread4(uint32_t b) {
+  return make_uint2((((b & 0xF) * 0x00204081u) & 0x01010101u) << 4, (((b >> 4) * 0x00204081u) & 0x01010101u) << 4);
+}
+// four nibbles (a byte each) through a 16-entry byte table in four registers
+__device__ __forceinline__ uint32_t table16(uint32_t n, const uint32_t (&t)[4]) {
+  const uint32_t s = n & 0x07070707u, lo = __builtin_amdgcn_perm(t[1], t[0], s), hi = __builtin_amdgcn_perm(t[3], t[2], s);
+  const uint32_t m = ((n >> 3) & 0x01010101u) * 0xFFu;
+  return (hi & m) | (lo & ~m);
+}
+__device__ __forceinline__ uint2 kvalues8(const uint2& n) {   // the IQ4 values + 128
+  uint32_t t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    t[i] = (uint32_t)(c_kvalues[4 * i] + 128) | ((uint32_t)(c_kvalues[4 * i + 1] + 128) << 8) |
+           ((uint32_t)(c_kvalues[4 * i + 2] + 128) << 16) | ((uint32_t)(c_kvalues[4 * i + 3] + 128) << 24);
+  return make_uint2(table16(n.x, t), table16(n.y, t));
 }
 
-// The 32 fp32 weights of group g (0..7) of the raw 256-weight record at rec.
-template <int T> __device__ void deq32(const uint8_t* rec, int g, float* w);
-
-template <> __device__ void deq32<GQK_Q4_0>(const uint8_t* rec, int g, float* w) {
-  const uint8_t* b = rec + 18 * g;
-  float d = f16_at(b);
-  for (int j = 0; j < 16; ++j) {
-    w[j] = d * (float)((int)(b[2 + j] & 0xF) - 8);
-    w[j + 16] = d * (float)((int)(b[2 + j] >> 4) - 8);
-  }
-}
-
-template <> __device__ void deq32<GQK_IQ4_NL>(const uint8_t* rec, int g, float* w) {
-  const uint8_t* b = rec + 18 * g;
-  float d = f16_at(b);
-  for (int j = 0; j < 16; ++j) {
-    w[j] = d * (float)c_kvalues[b[2 + j] & 0xF];
-    w[j + 16] = d * (float)c_kvalues[b[2 + j] >> 4];
-  }
-}
-
-template <> __device__ void deq32<GQK_Q5_0>(const uint8_t* rec, int g, float* w) {
-  const uint8_t* b = rec + 22 * g;
-  float d = f16_at(b);
-  uint32_t qh = (uint32_t)b[2] | ((uint32_t)b[3] << 8) | ((uint32_t)b[4] << 16) | ((uint32_t)b[5] << 24);
-  for (int j = 0; j < 16; ++j) {
-    int lo = (b[6 + j] & 0xF) | (((qh >> j) & 1) << 4);
-    int hi = (b[6 + j] >> 4) | (((qh >> (j + 16)) & 1) << 4);
-    w[j] = d * (float)(lo - 16);
-    w[j + 16] = d * (float)(hi - 16);
-  }
-}
-
-template <> __device__ void deq32<GQK_Q8_0>(const uint8_t* rec, int g, float* w) {
-  const uint8_t* b = rec + 34 * g;
-  float d = f16_at(b);
-  for (int j = 0; j < 32; ++j) w[j] = d * (float)(int8_t)b[2 + j];
-}
-
-template <> __device__ void deq32<GQK_Q2_K>(const uint8_t* rec, int g, float* w) {
-  // scales[16] | qs[64] | d | dmin; weight 128 h + 32 t + l = bits 2t of byte 32 h + l
-  float d = f16_at(rec + 80), dmin = f16_at(rec + 82);
-  int h = g >> 2, t = g & 3;
-  for (int hf = 0; hf < 2; ++hf) {
-    int sc = rec[8 * h + 2 * t + hf];
-    float dl = d * (float)(sc & 0xF), ml = dmin * (float)(sc >> 4);
-    for (int j = 0; j < 16; ++j) {
-      int l = 16 * hf + j;
-      int q = (rec[16 + 32 * h + l] >> (2 * t)) & 3;
-      w[l] = dl * (float)q - ml;
+// N fp32 weights of a record, from weight N i (N = 8 or 4).  q: eight integers in bytes, minus off;
+// w = dl * q, or dl * q - ml (K-quants with a min).  grid: the IQ3_S words in LDS.
+template <int T, int N, class S>
+__device__ __forceinline__ void decode(const S& s, int i, const uint32_t* grid, float (&w)[N]) {
+  const int e = N == 8 ? i : i >> 1;   // the eight weights 8 e .. that hold them
+  const int g = e >> 2, sub = e & 3;   // 32-weight group, eight of it
+  float dl, ml = 0.f, off = 0.f;
+  constexpr bool MIN = T == GQK_Q2_K || T == GQK_Q4_K || T == GQK_Q5_K;
+  uint2 q;
+  uint32_t qn[N / 4];   // the N integers
+  auto narrow = [&] {
+    if constexpr (N == 8) qn[0] = q.x, qn[1] = q.y;
+    else qn[0] = i & 1 ? q.y : q.x;
+  };
+  if constexpr (T == GQK_Q4_0 || T == GQK_IQ4_NL || T == GQK_Q5_0) {   // low nibbles: weights 0..15, high: 16..31
+    constexpr int PD = T == GQK_Q5_0 ? 2 : 1;
+    dl = f16_of(s.template ld<PD, uint16_t>(2 * g));
+    q = msk(s.template ld<0, uint2>(16 * g + 8 * (sub & 1)), 4 * (sub >> 1), 0x0F0F0F0Fu);
+    off = 8.f;
+    if constexpr (T == GQK_Q5_0) {
+      q = orr(q, spread4(s.template ld<1, uint8_t>(4 * g + sub)));
+      off = 16.f;
+    } else if constexpr (T == GQK_IQ4_NL) {
+      q = kvalues8(q);
+      off = 128.f;
     }
-  }
-}
-
-template <> __device__ void deq32<GQK_Q3_K>(const uint8_t* rec, int g, float* w) {
-  // hmask[32] | qs[64] | scales[12] | d   (kq_ref.py:40-56)
-  float d = f16_at(rec + 108);
-  const uint8_t* s = rec + 96;
-  int h = g >> 2, jj = g & 3;
-  for (int hf = 0; hf < 2; ++hf) {
-    int i = 2 * g + hf;
-    int lo = (s[i % 8] >> (4 * (i / 8))) & 0xF;
-    int hi = (s[8 + i % 4] >> (2 * (i / 4))) & 3;
-    float dl = d * (float)((lo | (hi << 4)) - 32);
-    for (int j = 0; j < 16; ++j) {
-      int l = 16 * hf + j;
-      int hb = (rec[l] >> (4 * h + jj)) & 1;
-      int q = ((rec[32 + 32 * h + l] >> (2 * jj)) & 3) - (hb ? 0 : 4);
-      w[l] = dl * (float)q;
+  } else if constexpr (T == GQK_Q8_0) {
+    dl = f16_of(s.template ld<1, uint16_t>(2 * g));
+    q = s.template ld<0, uint2>(32 * g + 8 * sub);
+    q.x ^= 0x80808080u, q.y ^= 0x80808080u;
+    off = 128.f;
+  } else if constexpr (T == GQK_Q2_K) {   // scales[16] | qs[64] | d | dmin; weight 128 h + 32 t + l = bits 2t of byte 32 h + l
+    const int h = g >> 2, t = g & 3;
+    const uint32_t dd = s.template ld<2, uint32_t>(0), sc = s.template ld<1, uint8_t>(8 * h + 2 * t + (sub >> 1));
+    dl = f16_of((uint16_t)dd) * (float)(sc & 0xF);
+    ml = f16_of((uint16_t)(dd >> 16)) * (float)(sc >> 4);
+    q = msk(s.template ld<0, uint2>(32 * h + 8 * sub), 2 * t, 0x03030303u);
+  } else if constexpr (T == GQK_Q3_K) {   // hmask[32] | qs[64] | scales[12] | d   (kq_ref.py:40-56)
+    const int h = g >> 2, jj = g & 3, k = 2 * g + (sub >> 1);
+    const int lo = (s.template ld<2, uint8_t>(k % 8) >> (4 * (k / 8))) & 0xF;
+    const int hi = (s.template ld<2, uint8_t>(8 + k % 4) >> (2 * (k / 4))) & 3;
+    dl = f16_of(s.template ld<3, uint16_t>(0)) * (float)((lo | (hi << 4)) - 32);
+    const uint2 hm = msk(s.template ld<1, uint2>(8 * sub), g, 0x01010101u);
+    q = orr(msk(s.template ld<0, uint2>(32 * h + 8 * sub), 2 * jj, 0x03030303u), make_uint2(hm.x << 2, hm.y << 2));
+    off = 4.f;
+  } else if constexpr (T == GQK_Q4_K || T == GQK_Q5_K) {   // d | dmin | scales[12] | (qh[32]) | qs[128]   (q4k.py:5-20, kq_ref.py:57-68)
+    constexpr int PH = T == GQK_Q4_K ? 1 : 2;
+    const uint32_t dd = s.template ld<PH, uint32_t>(0);
+    const uint32_t sa = s.template ld<PH, uint32_t>(4), sb = s.template ld<PH, uint32_t>(8), sv = s.template ld<PH, uint32_t>(12);
+    const int j = 8 * (g & 3);   // 6-bit scale and min of sub-block g (kq_ref.py:17-27)
+    const uint32_t a = (sa >> j) & 0xFF, b = (sb >> j) & 0xFF, c = (sv >> j) & 0xFF;
+    const int sc = g < 4 ? a & 63 : (c & 0xF) | ((a >> 6) << 4), m = g < 4 ? b & 63 : (c >> 4) | ((b >> 6) << 4);
+    dl = f16_of((uint16_t)dd) * (float)sc;
+    ml = f16_of((uint16_t)(dd >> 16)) * (float)m;
+    q = msk(s.template ld<0, uint2>(32 * (g >> 1) + 8 * sub), 4 * (g & 1), 0x0F0F0F0Fu);
+    if constexpr (T == GQK_Q5_K) {
+      const uint2 hb = msk(s.template ld<1, uint2>(8 * sub), g, 0x01010101u);
+      q = orr(q, make_uint2(hb.x << 4, hb.y << 4));
     }
-  }
-}
-
-template <int T> __device__ __forceinline__ void deq32_q45k(const uint8_t* rec, int g, float* w) {
-  // d | dmin | scales[12] | (qh[32]) | qs[128]   (q4k.py:5-20, kq_ref.py:57-68)
-  float d = f16_at(rec), dmin = f16_at(rec + 2);
-  int sc, m;
-  scale_min_k4(rec + 4, g, sc, m);
-  float dl = d * (float)sc, ml = dmin * (float)m;
-  const uint8_t* qs = rec + (T == GQK_Q4_K ? 16 : 48);
-  for (int p = 0; p < 32; ++p) {
-    int q = (qs[32 * (g >> 1) + p] >> (4 * (g & 1))) & 0xF;
-    if (T == GQK_Q5_K) q |= ((rec[16 + p] >> g) & 1) << 4;
-    w[p] = dl * (float)q - ml;
-  }
-}
-template <> __device__ void deq32<GQK_Q4_K>(const uint8_t* rec, int g, float* w) { deq32_q45k<GQK_Q4_K>(rec, g, w); }
-template <> __device__ void deq32<GQK_Q5_K>(const uint8_t* rec, int g, float* w) { deq32_q45k<GQK_Q5_K>(rec, g, w); }
-
-template <> __device__ void deq32<GQK_Q6_K>(const uint8_t* rec, int g, float* w) {
-  // ql[128] | qh[64] | int8 scales[16] | d   (kq_ref.py:69-79)
-  float d = f16_at(rec + 208);
-  int h = g >> 2, t = g & 3;
-  for (int hf = 0; hf < 2; ++hf) {
-    float dl = d * (float)(int8_t)rec[192 + 8 * h + 2 * t + hf];
-    for (int j = 0; j < 16; ++j) {
-      int p = 16 * hf + j;
-      int lo = (rec[64 * h + 32 * (t & 1) + p] >> (4 * (t >> 1))) & 0xF;
-      int hi = (rec[128 + 32 * h + p] >> (2 * t)) & 3;
-      w[p] = dl * (float)((lo | (hi << 4)) - 32);
+  } else if constexpr (T == GQK_Q6_K) {   // ql[128] | qh[64] | int8 scales[16] | d   (kq_ref.py:69-79)
+    const int g16 = e >> 1;
+    dl = f16_of(s.template ld<2, uint16_t>(0)) * (float)(int8_t)s.template ld<1, uint8_t>(g16);
+    if constexpr (S::PACKED6) {   // the six-bit values re-packed per scale group (gqk_q6_pos)
+      uint32_t P[3];
+#pragma unroll
+      for (int m = 0; m < 3; ++m) P[m] = s.template ld<0, uint32_t>(gqk_q6_pos(g16, m, 0));
+      const uint32_t top = ((P[0] >> 6) & 0x03030303u) | ((P[1] >> 4) & 0x0C0C0C0Cu) | ((P[2] >> 2) & 0x30303030u);
+      q = e & 1 ? make_uint2(P[2] & 0x3F3F3F3Fu, top) : make_uint2(P[0] & 0x3F3F3F3Fu, P[1] & 0x3F3F3F3Fu);
+    } else {
+      const int h = g >> 2, t = g & 3;
+      const uint2 hi = msk(s.template raw<uint2>(128 + 32 * h + 8 * sub), 2 * t, 0x03030303u);
+      q = orr(msk(s.template raw<uint2>(64 * h + 32 * (t & 1) + 8 * sub), 4 * (t >> 1), 0x0F0F0F0Fu), make_uint2(hi.x << 4, hi.y << 4));
     }
-  }
-}
-
-template <> __device__ void deq32<GQK_IQ4_XS>(const uint8_t* rec, int g, float* w) {
-  // d | scales_h u16 | scales_l[4] | qs[128]   (iq4xs.py:5-11)
-  float d = f16_at(rec);
-  int sh = rec[2] | (rec[3] << 8);
-  int ls = ((rec[4 + g / 2] >> (4 * (g % 2))) & 0xF) | (((sh >> (2 * g)) & 3) << 4);
-  float dl = d * (float)(ls - 32);
-  const uint8_t* qs = rec + 8 + 16 * g;
-  for (int j = 0; j < 16; ++j) {
-    w[j] = dl * (float)c_kvalues[qs[j] & 0xF];
-    w[j + 16] = dl * (float)c_kvalues[qs[j] >> 4];
-  }
-}
-
-template <> __device__ void deq32<GQK_IQ3_S>(const uint8_t* rec, int g, float* w) {
-  // d | qs[64] | qh[8] | signs[32] | scales[4]   (iq3s_tile_dequant.py:30-53)
-  float d = f16_at(rec);
-  int s = (rec[106 + g / 2] >> (4 * (g % 2))) & 0xF;
-  float dl = d * (float)(1 + 2 * s);
-  int qh = rec[66 + g];
-  for (int l = 0; l < 4; ++l) {
-    int sg = rec[74 + 4 * g + l];
-    for (int half = 0; half < 2; ++half) {
-      int idx = rec[2 + 8 * g + 2 * l + half] | ((qh << (8 - 2 * l - half)) & 256);
-      uint32_t gw = c_iq3s_grid[idx];
-      for (int k4 = 0; k4 < 4; ++k4) {
-        int jj = 4 * half + k4;
-        float v = dl * (float)((gw >> (8 * k4)) & 0xFF);
-        w[8 * l + jj] = ((sg >> jj) & 1) ? -v : v;
-      }
+    off = 32.f;
+  } else if constexpr (T == GQK_IQ4_XS) {   // d | scales_h u16 | scales_l[4] | qs[128]   (iq4xs.py:5-11)
+    const uint32_t dd = s.template ld<1, uint32_t>(0);
+    const int ls = ((s.template ld<1, uint8_t>(4 + g / 2) >> (4 * (g % 2))) & 0xF) | (((dd >> (16 + 2 * g)) & 3) << 4);
+    dl = f16_of((uint16_t)dd) * (float)(ls - 32);
+    q = kvalues8(msk(s.template ld<0, uint2>(16 * g + 8 * (sub & 1)), 4 * (sub >> 1), 0x0F0F0F0Fu));
+    off = 128.f;
+  } else {   // IQ3_S: d | qs[64] | qh[8] | signs[32] | scales[4]   (iq3s_tile_dequant.py:30-53)
+    static_assert(T == GQK_IQ3_S, "type");
+    const int sc = (s.template ld<3, uint8_t>(g / 2) >> (4 * (g % 2))) & 0xF;
+    dl = f16_of(s.template ld<4, uint16_t>(0)) * (float)(1 + 2 * sc);
+    const uint32_t qs = s.template ld<0, uint16_t>(8 * g + 2 * sub), qh = s.template ld<2, uint8_t>(g), sg = s.template ld<1, uint8_t>(4 * g + sub);
+    q = make_uint2(grid[(qs & 0xFF) | ((qh << (8 - 2 * sub)) & 256)], grid[(qs >> 8) | ((qh << (7 - 2 * sub)) & 256)]);
+    narrow();
+    const uint32_t sn = N == 8 ? sg : sg >> (4 * (i & 1));
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float v = dl * ub<N>(qn, j);
+      w[j] = (sn >> j) & 1 ? -v : v;
     }
+    return;
+  }
+  narrow();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float v = ub<N>(qn, j) - off;   // an exact integer
+    w[j] = MIN ? dl * v - ml : dl * v;
   }
 }
 
@@ -179,46 +190,73 @@ template <> __device__ __forceinline__ _Float16 cvt_out<_Float16>(float v) {
   return (_Float16)v;
 }
 
-// One thread per (row, group of 32 weights).  VEC: the output rows are 16-byte aligned, so the
-// 32 values go out as 16-byte stores (64 or 128 contiguous bytes per thread).
-template <int T, typename O, bool VEC>
-__global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ W, int64_t stride, int64_t n,
-                                                      int64_t K, O* __restrict__ out, int64_t ldo, int rec) {
-  int64_t ng = K / 32;
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * ng) return;
-  int64_t row = i / ng, gg = i % ng;
-  int64_t kb = gg / 8;
-  int g = (int)(gg % 8);
-  const uint8_t* recp = W + row * stride + kb * rec;
-  float w[32];
-  deq32<T>(recp, g, w);
-  O* o = out + row * ldo + gg * 32;
+// N values to their place: one 16-byte store where the rows allow it (VEC)
+template <typename O, bool VEC, int N>
+__device__ __forceinline__ void store_n(O* o, const float (&w)[N]) {
+  static_assert(N * sizeof(O) == 16, "16 bytes a thread");
+  O c[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) c[j] = cvt_out<O>(w[j]);
   if constexpr (VEC) {
-    constexpr int PER = 16 / sizeof(O);   // values per 16-byte store
-    uint4* ov = (uint4*)o;
-#pragma unroll
-    for (int v = 0; v < 32 / PER; ++v) {
-      O c[PER];
-#pragma unroll
-      for (int j = 0; j < PER; ++j) c[j] = cvt_out<O>(w[v * PER + j]);
-      ov[v] = __builtin_bit_cast(uint4, c);
-    }
+    *(uint4*)o = __builtin_bit_cast(uint4, c);
   } else {
 #pragma unroll
-    for (int j = 0; j < 32; ++j) o[j] = cvt_out<O>(w[j]);
+    for (int j = 0; j < N; ++j) o[j] = c[j];
+  }
+}
+
+#define DQ_ITEMS 4                    // items per thread
+#define DQ_SPAN (256 * DQ_ITEMS)      // items per workgroup
+template <int T> __device__ __forceinline__ const uint32_t* iq3s_grid(uint32_t* lds) {
+  if constexpr (T == GQK_IQ3_S) {
+    for (int t = threadIdx.x; t < 512; t += 256) lds[t] = c_iq3s_grid[t];
+    __syncthreads();
+  }
+  return lds;
+}
+
+// One item = 16 output bytes (eight 16-bit weights, four fp32 ones) of a row, consecutive threads
+// consecutive items, so that a wave writes 1 KiB of whole lines and its reads of a record fall in a few
+// lines.  Bound by the writes (bf16: 3.5 bytes out per byte of Q4_K in); 34816 x 5120 from 32 weights a
+// thread (byte reads, stores 64 bytes apart) -> this, us: bf16 Q4_K 169 -> 108, Q6_K 146 -> 100, Q8_0
+// 145 -> 95, Q4_0 137 -> 84, IQ4_XS 165 -> 83, IQ3_S 150 -> 101.  magic = ceil(2^32 / items per row).
+template <int T, typename O, bool VEC>
+__global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ W, int64_t stride, int64_t n,
+                                                      int64_t K, O* __restrict__ out, int64_t ldo, uint32_t magic) {
+  __shared__ uint32_t lds[T == GQK_IQ3_S ? 512 : 1];
+  const uint32_t* grid = iq3s_grid<T>(lds);
+  constexpr int N = 16 / sizeof(O), IR = 256 / N;   // weights per item, items per record
+  const int64_t ipr = K / N, base = (int64_t)blockIdx.x * DQ_SPAN;
+  const int64_t row0 = base / ipr, rem0 = base - row0 * ipr;
+#pragma unroll
+  for (int k = 0; k < DQ_ITEMS; ++k) {
+    const uint32_t d = k * 256 + threadIdx.x;
+    int64_t row = row0, it = rem0 + d;
+    if (ipr >= DQ_SPAN) {
+      if (it >= ipr) it -= ipr, ++row;
+    } else {   // it < 2 DQ_SPAN: the product with magic is exact
+      const uint32_t r = __umulhi((uint32_t)it, magic);
+      row += r;
+      it -= (int64_t)(r * (uint32_t)ipr);
+    }
+    if (row >= n) return;
+    const RawSrc<T> s{W + row * stride + it / IR * gqk_layout<T>::REC};
+    float w[N];
+    decode<T, N>(s, (int)(it % IR), grid, w);
+    store_n<O, VEC, N>(out + row * ldo + it * N, w);
   }
 }
 
 template <int T>
 static int launch_dequant_t(const void* W, int64_t stride, int64_t n, int64_t K, void* out, int64_t ldo, int dtype,
                             hipStream_t st) {
-  const int rec = gqk_layout<T>::REC;
-  int64_t total = n * (K / 32);
-  dim3 grid((unsigned)((total + 255) / 256)), block(256);
+  const int64_t ipr = K / (dtype == 0 ? 4 : 8), wgs = (n * ipr + DQ_SPAN - 1) / DQ_SPAN;
+  if (wgs >= ((int64_t)1 << 31)) return GQK_ERR_SHAPE;
+  const dim3 grid((unsigned)wgs), block(256);
+  const uint32_t magic = (uint32_t)(((1ull << 32) + ipr - 1) / ipr);
   const int esz = dtype == 0 ? 4 : 2;
   const bool vec = ((uintptr_t)out % 16 == 0) && ((ldo * esz) % 16 == 0);
-#define L(O, V) hipLaunchKernelGGL((dequant_kernel<T, O, V>), grid, block, 0, st, (const uint8_t*)W, stride, n, K, (O*)out, ldo, rec)
+#define L(O, V) hipLaunchKernelGGL((dequant_kernel<T, O, V>), grid, block, 0, st, (const uint8_t*)W, stride, n, K, (O*)out, ldo, magic)
   if (dtype == 0) {
     if (vec) L(float, true); else L(float, false);
   } else if (dtype == 1) {
@@ -249,20 +287,6 @@ int launch_dequant(int type, const void* W, int64_t stride, int64_t n, int64_t K
 // back row by row.  Rows past n are zeros in the tiles (repack) and are not written (unrepack).
 // Each byte crosses HBM once in each direction.  The plane table is a compile-time constant per
 // type, so the index arithmetic folds to shifts and multiplies by constants.
-
-// raw byte of byte j of plane p (segments of equal length concatenated)
-template <int T, int P>
-__device__ __forceinline__ int raw_of(int j) {
-  constexpr gqk_plane pl = gqk_planes<T>::v.planes[P];
-  return pl.seg_off + (j / pl.seg_len) * pl.seg_stride + j % pl.seg_len;
-}
-
-template <int T, int P>
-__device__ __forceinline__ constexpr int plane_off() {
-  int o = 0;
-  for (int p = 0; p < P; ++p) o += gqk_planes<T>::v.planes[p].size;
-  return o;
-}
 
 // visits the 16-byte words of plane P of a chunk: f(word index in the chunk, row of byte i, raw
 // byte of byte i) for i = 0..15 through g(i) -> (r, b)
@@ -348,9 +372,8 @@ __device__ __forceinline__ void q6_convert(uint8_t* raw, int tid) {
 }
 
 // The 64 raw records of a chunk from its plane-major words (16-byte loads), into raw[row][REC] in
-// LDS (Q6_K's six-bit values converted back to ql / qh before the function returns, unless
-// Q6_PACKED: then its first 192 bytes stay in the re-packed order).
-template <int T, bool Q6_PACKED = false>
+// LDS (Q6_K's six-bit values converted back to ql / qh before the function returns).
+template <int T>
 __device__ __forceinline__ void chunk_to_raw(const uint4* __restrict__ in, uint8_t* raw, int tid) {
   constexpr int REC = gqk_planes<T>::v.rec;
   auto scatter = [&](int wi, auto&& at) {
@@ -364,31 +387,9 @@ __device__ __forceinline__ void chunk_to_raw(const uint4* __restrict__ in, uint8
     }
   };
   every_plane_word<T>(tid, scatter);
-  if constexpr (T == GQK_Q6_K && !Q6_PACKED) {
+  if constexpr (T == GQK_Q6_K) {
     __syncthreads();
     q6_convert<false>(raw, tid);
-  }
-}
-
-// deq32<Q6_K> on a record whose six-bit values are in the re-packed order (gqk_q6_pos): the same
-// weights and the same fp32 bits, without restoring ql / qh first.
-__device__ __forceinline__ void deq32_q6_packed(const uint8_t* rec, int g, float* w) {
-  const float d = f16_at(rec + 208);
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const int g16 = 2 * g + hf;
-    const float dl = d * (float)(int8_t)rec[192 + g16];
-    uint32_t top[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t b = rec[gqk_q6_pos(g16, m, i)];
-        w[16 * hf + 4 * m + i] = dl * (float)((int)(b & 63) - 32);
-        top[i] |= (b >> 6) << (2 * m);
-      }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[16 * hf + 12 + i] = dl * (float)((int)top[i] - 32);
   }
 }
 
@@ -483,41 +484,36 @@ int launch_repack(int type, const void* W, int64_t stride, int64_t n, int64_t K,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Dequantize straight from the tiles: one workgroup per chunk (tile t, super-block kb) gathers the
-// chunk's planes back into its 64 raw records in LDS (as the unrepack does), then every thread
-// decodes (row, 32-weight group) items from LDS with the same deq32 as the raw-row dequantizer
-// and writes them to the output row: each tile byte is read once, no raw-row temporary.
+// Dequantize straight from the tiles: one workgroup per chunk (tile t, super-block kb) copies the chunk
+// to LDS as it lies, then decodes items of 16 output bytes from its planes.  A wave takes eight rows x
+// eight items: 128 bytes per row, whole lines.  Each tile byte is read once.  34816 x 5120 to bf16 from
+// the chunk scattered back to raw records byte by byte -> this, us: Q4_K 129 -> 83, Q6_K 148 -> 94, Q8_0
+// 151 -> 106, IQ4_XS 171 -> 85, IQ3_S 153 -> 82 (5.2-5.5 TB/s read + written).
 template <int T, typename O, bool VEC>
 __global__ __launch_bounds__(256) void tile_dequant_kernel(const uint8_t* __restrict__ tiles, int64_t n, int64_t nb,
                                                            O* __restrict__ out, int64_t ldo) {
   constexpr int REC = gqk_planes<T>::v.rec, CB = 64 * REC;
-  __shared__ __attribute__((aligned(16))) uint8_t raw[CB + 16];
+  constexpr int N = 16 / sizeof(O), IP = 32 / N;   // weights per item, passes of eight items per row
+  __shared__ __attribute__((aligned(16))) uint8_t raw[CB];
+  __shared__ uint32_t lds[T == GQK_IQ3_S ? 512 : 1];
   const int tid = threadIdx.x;
   const int64_t chunk = blockIdx.x, kb = chunk % nb, tile = chunk / nb;
-  chunk_to_raw<T, true>((const uint4*)(tiles + chunk * CB), raw, tid);
+  const uint4* in = (const uint4*)(tiles + chunk * CB);
+#pragma unroll
+  for (int k = 0; k < (CB / 16 + 255) / 256; ++k) {
+    const int i = k * 256 + tid;
+    if (i < CB / 16) ((uint4*)raw)[i] = in[i];
+  }
+  const uint32_t* grid = iq3s_grid<T>(lds);
   __syncthreads();
-  for (int it = tid; it < 64 * 8; it += 256) {   // consecutive threads: consecutive groups of a row
-    const int r = it >> 3, g = it & 7;
-    const int64_t row = tile * 64 + r;
-    if (row >= n) continue;
-    float w[32];
-    if constexpr (T == GQK_Q6_K) deq32_q6_packed(raw + r * REC, g, w);
-    else deq32<T>(raw + r * REC, g, w);
-    O* o = out + row * ldo + kb * 256 + g * 32;
-    if constexpr (VEC) {
-      constexpr int PER = 16 / sizeof(O);
-      uint4* ov = (uint4*)o;
+  const int64_t rows = n - tile * 64;
 #pragma unroll
-      for (int v = 0; v < 32 / PER; ++v) {
-        O c[PER];
-#pragma unroll
-        for (int j = 0; j < PER; ++j) c[j] = cvt_out<O>(w[v * PER + j]);
-        ov[v] = __builtin_bit_cast(uint4, c);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 32; ++j) o[j] = cvt_out<O>(w[j]);
-    }
+  for (int k = 0; k < 2 * IP; ++k) {   // pass k: rows 32 (k / IP) + 8 wave + lane / 8, items 8 (k % IP) + lane % 8
+    const int r = 32 * (k / IP) + 8 * (tid >> 6) + ((tid & 63) >> 3), e = 8 * (k % IP) + (tid & 7);
+    if (r >= rows) continue;
+    float w[N];
+    decode<T, N>(TileSrc<T>{raw, r}, e, grid, w);
+    store_n<O, VEC, N>(out + (tile * 64 + r) * ldo + kb * 256 + e * N, w);
   }
 }
 
