@@ -280,13 +280,10 @@ int launch_dequant(int type, const void* W, int64_t stride, int64_t n, int64_t K
 }
 
 // ---------------------------------------------------------------------------------------------
-// Repack raw rows <-> tiles.  One workgroup per chunk (tile t, super-block kb): 64 rows x REC bytes.
-// Repack stages the chunk's 64 raw records in LDS (2-byte loads along each row when the rows are
-// 2-byte aligned, REC being even) and writes the chunk plane-major with 16-byte stores; unrepack
-// loads the chunk with 16-byte loads, scatters it into the 64 raw records in LDS and writes them
-// back row by row.  Rows past n are zeros in the tiles (repack) and are not written (unrepack).
-// Each byte crosses HBM once in each direction.  The plane table is a compile-time constant per
-// type, so the index arithmetic folds to shifts and multiplies by constants.
+// Repack raw rows <-> tiles.  One workgroup per chunk (tile t, super-block kb): 64 rows x REC bytes,
+// through the 64 raw records in LDS.  Rows past n are zeros in the tiles (repack) and are not written
+// (unrepack).  Each byte crosses HBM once in each direction.  The plane table is a compile-time constant
+// per type, so the index arithmetic folds to shifts and multiplies by constants.
 
 // visits the 16-byte words of plane P of a chunk: f(word index in the chunk, row of byte i, raw
 // byte of byte i) for i = 0..15 through g(i) -> (r, b)
@@ -312,13 +309,6 @@ __device__ __forceinline__ void every_plane_word(int tid, F&& f) {
 }
 
 // ---- Q6_K: the six-bit values re-packed per scale group (gqk_q6_pos) <-> GGUF's ql / qh ----------
-// q of weight k of a raw record (ql[128] | qh[64], kq_ref.py:69-79): 4 low bits from ql, 2 from qh
-__device__ __forceinline__ uint32_t q6_raw(const uint8_t* rec, int k) {
-  const int hh = k >> 7, l = k & 127;
-  const uint32_t lo = (rec[64 * hh + (l & 63)] >> (4 * (l >> 6))) & 0xF;
-  const uint32_t hi = (rec[128 + 32 * hh + (l & 31)] >> (2 * (l >> 5))) & 3;
-  return lo | (hi << 4);
-}
 // q of weight k of a re-packed record
 __device__ __forceinline__ uint32_t q6_packed(const uint8_t* rec, int k) {
   const int g = k >> 4, j = k & 15;
@@ -328,10 +318,8 @@ __device__ __forceinline__ uint32_t q6_packed(const uint8_t* rec, int k) {
   for (int m = 0; m < 3; ++m) v |= (uint32_t)(rec[gqk_q6_pos(g, m, j - 12)] >> 6) << (2 * m);
   return v;
 }
-// In place on the chunk's 64 records in LDS (raw[row][REC]): TO_PACKED re-packs bytes 0..191 of
-// every record, else restores GGUF's ql / qh.  Every thread computes its share into registers
+// In place on the chunk's 64 records in LDS (raw[row][REC]): restores GGUF's ql / qh.  Every thread computes its share into registers
 // before any is written (barriers between), so the pass reads only the old layout.
-template <bool TO_PACKED>
 __device__ __forceinline__ void q6_convert(uint8_t* raw, int tid) {
   constexpr int REC = 210, PER = 64 * 48 / 256;   // 48 dwords of 192 bytes per row, 12 per thread
   uint32_t v[PER];
@@ -344,10 +332,7 @@ __device__ __forceinline__ void q6_convert(uint8_t* raw, int tid) {
     for (int i = 0; i < 4; ++i) {
       const int b = 4 * w + i;   // output byte
       uint32_t byte;
-      if (TO_PACKED) {             // byte b = gqk_q6_pos(g, m, i'): low 6 bits of q[16 g + 4 m + i'], top 2 of q[16 g + 12 + i']
-        const int col = b >> 4, a = col / 3, m = col % 3, g = 4 * a + ((b >> 2) & 3), ii = b & 3;
-        byte = (q6_raw(rec, 16 * g + 4 * m + ii) & 63) | (((q6_raw(rec, 16 * g + 12 + ii) >> (2 * m)) & 3) << 6);
-      } else if (b < 128) {        // ql byte b: low nibbles of weights 128 hh + p and 128 hh + 64 + p
+      if (b < 128) {               // ql byte b: low nibbles of weights 128 hh + p and 128 hh + 64 + p
         const int hh = b >> 6, p = b & 63;
         byte = (q6_packed(rec, 128 * hh + p) & 15) | ((q6_packed(rec, 128 * hh + 64 + p) & 15) << 4);
       } else {                     // qh byte: the high pairs of weights 128 hh + p + 32 t
@@ -389,76 +374,163 @@ __device__ __forceinline__ void chunk_to_raw(const uint4* __restrict__ in, uint8
   every_plane_word<T>(tid, scatter);
   if constexpr (T == GQK_Q6_K) {
     __syncthreads();
-    q6_convert<false>(raw, tid);
+    q6_convert(raw, tid);
   }
 }
 
-template <int T, bool TO_TILES, bool WIDE>
+// Bytes o .. o + U - 1 (o even) of an LDS row whose base is 16-byte aligned: whole dwords and a byte shift.
+template <int U>
+__device__ __forceinline__ void lds_bytes(const uint8_t* row, int o, uint32_t* d) {
+  if constexpr (U == 2) {
+    d[0] = *(const uint16_t*)(row + o);
+  } else {
+    const uint32_t* p = (const uint32_t*)(row + (o & ~3));
+    uint32_t v[U / 4 + 1];
+#pragma unroll
+    for (int i = 0; i <= U / 4; ++i) v[i] = p[i];
+#pragma unroll
+    for (int i = 0; i < U / 4; ++i) d[i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], o & 3);
+  }
+}
+// Writes plane P of a chunk from the 64 raw records in LDS (row stride RS): every 16-byte word is made of
+// units that are contiguous in the record.
+template <int T, int P, int RS>
+__device__ __forceinline__ void write_plane(const uint8_t* raw, uint4* out, int tid) {
+  constexpr gqk_plane pl = gqk_planes<T>::v.planes[P];
+  constexpr int W = gqk_col_width(pl.size), U = W < pl.seg_len ? W : pl.seg_len < 16 ? pl.seg_len : 16;
+  static_assert(U == 2 || U == 4 || U == 8 || U == 16, "unit");
+  for (int w = tid; w < 4 * pl.size; w += 256) {     // 64 rows * size bytes / 16
+    const int x = 16 * w, col = x / (64 * W), rem = x % (64 * W);
+    uint32_t d[4];
+    if constexpr (U == 2) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t u[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int b = rem + 4 * i + 2 * k;
+          lds_bytes<2>(raw + b / W * RS, raw_of<T, P>(col * W + b % W), u + k);
+        }
+        d[i] = u[0] | (u[1] << 16);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16 / U; ++i) {
+        const int b = rem + U * i;
+        lds_bytes<U>(raw + b / W * RS, raw_of<T, P>(col * W + b % W), d + U / 4 * i);
+      }
+    }
+    out[4 * plane_off<T, P>() + w] = make_uint4(d[0], d[1], d[2], d[3]);
+  }
+}
+// Q6_K's first plane: the six-bit values re-packed per scale group (gqk_q6_pos), four at a time.  q of
+// weights k .. k + 3 (k % 4 = 0) of a raw record: four low bits from ql, two from qh.
+__device__ __forceinline__ uint32_t q6_raw4(const uint8_t* rec, int k) {
+  const int hh = k >> 7, t = (k >> 5) & 3, p = k & 31;
+  const uint32_t lo = *(const uint32_t*)(rec + 64 * hh + 32 * (t & 1) + p) >> (4 * (t >> 1));
+  const uint32_t hi = *(const uint32_t*)(rec + 128 + 32 * hh + p) >> (2 * t);
+  return (lo & 0x0F0F0F0Fu) | ((hi & 0x03030303u) << 4);
+}
+template <int RS>
+__device__ __forceinline__ void write_plane_q6(const uint8_t* raw, uint4* out, int tid) {
+  for (int w = tid; w < 4 * 192; w += 256) {
+    const int col = w >> 6, a = col / 3, m = col % 3;
+    const uint8_t* rec = raw + (w & 63) * RS;
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = 16 * (4 * a + i);
+      d[i] = q6_raw4(rec, k + 4 * m) | (((q6_raw4(rec, k + 12) >> (2 * m)) & 0x03030303u) << 6);
+    }
+    out[w] = make_uint4(d[0], d[1], d[2], d[3]);
+  }
+}
+template <int T, int P, int RS>
+__device__ __forceinline__ void write_planes(const uint8_t* raw, uint4* out, int tid) {
+  if constexpr (P < gqk_planes<T>::v.nplanes) {
+    if constexpr (T == GQK_Q6_K && P == 0) write_plane_q6<RS>(raw, out, tid);
+    else write_plane<T, P, RS>(raw, out, tid);
+    write_planes<T, P + 1, RS>(raw, out, tid);
+  }
+}
+
+// Raw rows -> tiles, bound by HBM.  The chunk's 64 records go to LDS by 16-byte loads of any alignment
+// (the last one of a record overlaps the one before and is shifted into place), all in flight before
+// the first is stored, and the planes come back by dwords.  Workgroup b runs on XCD b % 8, which takes
+// a contiguous range of chunks: consecutive super-blocks of a row share 128-byte lines, and each XCD's
+// L2 then fetches them once.
+// 34816 x 5120 from 2-byte row loads and byte gathers -> this, us: Q4_K 76 -> 37, Q6_K 198 -> 57 (its
+// six-bit values went byte by byte through a second pass), Q8_0 148 -> 73, Q5_K 93 -> 44, IQ4_XS 72 -> 35,
+// Q2_K 36 -> 18 (5.1-6.4 TB/s read + written).
+template <int T>
 __global__ __launch_bounds__(256) void repack_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                     int64_t stride, int64_t n, int64_t nb) {
-  constexpr gqk_type_c ty = gqk_planes<T>::v;
-  constexpr int REC = ty.rec, CB = 64 * REC;          // chunk bytes (a multiple of 64)
+                                                     int64_t stride, int64_t n, int64_t nb, int64_t chunks) {
+  constexpr int REC = gqk_planes<T>::v.rec, NV = REC / 16, TAIL = REC % 16, NT = NV + (TAIL != 0);
+  constexpr int RS = 16 * NT, IT = (64 * NT + 255) / 256;
+  __shared__ __attribute__((aligned(16))) uint8_t raw[64 * RS + 16];
+  const int tid = threadIdx.x;
+  const int64_t per = (chunks + 7) / 8, chunk = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || chunk >= chunks) return;
+  const int64_t kb = chunk % nb, row0 = chunk / nb * 64;
+  const uint8_t* rows = src + row0 * stride + kb * REC;
+  uint4 v[IT];
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int i = k * 256 + tid, r = i / NT, c = i % NT;
+    v[k] = make_uint4(0, 0, 0, 0);
+    if (i < 64 * NT && row0 + r < n) v[k] = load_any<uint4>(rows + r * stride + (c < NV ? 16 * c : REC - 16));
+  }
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int i = k * 256 + tid, r = i / NT, c = i % NT;
+    uint4 q = v[k];
+    if (TAIL != 0 && c == NV) {   // bytes 16 - TAIL .. 15 of the load belong at byte 16 NV
+      constexpr int sh = 16 - TAIL, sd = sh / 4, sb = sh % 4;
+      const uint32_t s[9] = {q.x, q.y, q.z, q.w, 0, 0, 0, 0, 0};
+      q = make_uint4(__builtin_amdgcn_alignbyte(s[sd + 1], s[sd], sb), __builtin_amdgcn_alignbyte(s[sd + 2], s[sd + 1], sb),
+                     __builtin_amdgcn_alignbyte(s[sd + 3], s[sd + 2], sb), __builtin_amdgcn_alignbyte(s[sd + 4], s[sd + 3], sb));
+    }
+    if (i < 64 * NT) *(uint4*)(raw + r * RS + 16 * c) = q;
+  }
+  __syncthreads();
+  write_planes<T, 0, RS>(raw, (uint4*)(dst + chunk * (64 * REC)), tid);
+}
+
+// Tiles -> raw rows
+template <int T, bool WIDE>
+__global__ __launch_bounds__(256) void unrepack_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
+                                                       int64_t stride, int64_t n, int64_t nb) {
+  constexpr int REC = gqk_planes<T>::v.rec, CB = 64 * REC;          // chunk bytes (a multiple of 64)
   __shared__ __attribute__((aligned(16))) uint8_t raw[CB + 16];   // the 64 raw records, [row][REC]
   const int tid = threadIdx.x;
   const int64_t chunk = blockIdx.x, kb = chunk % nb, tile = chunk / nb;
   const int64_t row0 = tile * 64;
-  if (TO_TILES) {
-    const uint8_t* rows = src + row0 * stride + kb * REC;
-    if (WIDE) {
-      for (int i = tid; i < CB / 2; i += 256) {
-        const int r = i / (REC / 2), h = i % (REC / 2);
-        const uint16_t v = row0 + r < n ? *(const uint16_t*)(rows + r * stride + 2 * h) : (uint16_t)0;
-        *(uint16_t*)(raw + r * REC + 2 * h) = v;
-      }
-    } else {
-      for (int i = tid; i < CB; i += 256) {
-        const int r = i / REC, b = i % REC;
-        raw[i] = row0 + r < n ? rows[r * stride + b] : (uint8_t)0;
-      }
+  chunk_to_raw<T>((const uint4*)(src + chunk * CB), raw, tid);
+  __syncthreads();
+  uint8_t* rows = dst + row0 * stride + kb * REC;
+  if (WIDE) {
+    for (int i = tid; i < CB / 2; i += 256) {
+      const int r = i / (REC / 2), h = i % (REC / 2);
+      if (row0 + r < n) *(uint16_t*)(rows + r * stride + 2 * h) = *(const uint16_t*)(raw + r * REC + 2 * h);
     }
-    __syncthreads();
-    if constexpr (T == GQK_Q6_K) q6_convert<true>(raw, tid);
-    uint4* out = (uint4*)(dst + chunk * CB);
-    auto gather = [&](int wi, auto&& at) {
-      uint32_t v[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        int r, b;
-        at(i, r, b);
-        v[i >> 2] |= (uint32_t)raw[r * REC + b] << (8 * (i & 3));
-      }
-      out[wi] = make_uint4(v[0], v[1], v[2], v[3]);
-    };
-    every_plane_word<T>(tid, gather);
   } else {
-    chunk_to_raw<T>((const uint4*)(src + chunk * CB), raw, tid);
-    __syncthreads();
-    uint8_t* rows = dst + row0 * stride + kb * REC;
-    if (WIDE) {
-      for (int i = tid; i < CB / 2; i += 256) {
-        const int r = i / (REC / 2), h = i % (REC / 2);
-        if (row0 + r < n) *(uint16_t*)(rows + r * stride + 2 * h) = *(const uint16_t*)(raw + r * REC + 2 * h);
-      }
-    } else {
-      for (int i = tid; i < CB; i += 256) {
-        const int r = i / REC, b = i % REC;
-        if (row0 + r < n) rows[r * stride + b] = raw[i];
-      }
+    for (int i = tid; i < CB; i += 256) {
+      const int r = i / REC, b = i % REC;
+      if (row0 + r < n) rows[r * stride + b] = raw[i];
     }
   }
 }
 
 template <int T>
-static void launch_repack_t(bool to_tiles, bool wide, dim3 grid, hipStream_t st, const uint8_t* s, uint8_t* d,
+static void launch_repack_t(bool to_tiles, bool wide, int64_t chunks, hipStream_t st, const uint8_t* s, uint8_t* d,
                             int64_t stride, int64_t n, int64_t nb) {
   const dim3 block(256);
-  if (to_tiles) {
-    if (wide) hipLaunchKernelGGL((repack_kernel<T, true, true>), grid, block, 0, st, s, d, stride, n, nb);
-    else hipLaunchKernelGGL((repack_kernel<T, true, false>), grid, block, 0, st, s, d, stride, n, nb);
-  } else {
-    if (wide) hipLaunchKernelGGL((repack_kernel<T, false, true>), grid, block, 0, st, s, d, stride, n, nb);
-    else hipLaunchKernelGGL((repack_kernel<T, false, false>), grid, block, 0, st, s, d, stride, n, nb);
-  }
+  if (to_tiles)
+    hipLaunchKernelGGL((repack_kernel<T>), dim3((unsigned)((chunks + 7) / 8 * 8)), block, 0, st, s, d, stride, n, nb, chunks);
+  else if (wide)
+    hipLaunchKernelGGL((unrepack_kernel<T, true>), dim3((unsigned)chunks), block, 0, st, s, d, stride, n, nb);
+  else
+    hipLaunchKernelGGL((unrepack_kernel<T, false>), dim3((unsigned)chunks), block, 0, st, s, d, stride, n, nb);
 }
 
 int launch_repack(int type, const void* W, int64_t stride, int64_t n, int64_t K, void* tiles, bool to_tiles,
@@ -469,13 +541,12 @@ int launch_repack(int type, const void* W, int64_t stride, int64_t n, int64_t K,
   const int64_t chunks = ntiles * nb;
   if (chunks == 0) return GQK_OK;
   if (chunks >= ((int64_t)1 << 31)) return GQK_ERR_SHAPE;
-  // 2-byte accesses along the raw rows when every row starts 2-byte aligned (every REC is even)
+  // unrepack: 2-byte accesses along the raw rows when every row starts 2-byte aligned (every REC is even)
   const bool wide = (t->rec % 2 == 0) && (stride % 2 == 0) && ((uintptr_t)W % 2 == 0);
-  const dim3 grid((unsigned)chunks);
   const uint8_t* s = (const uint8_t*)(to_tiles ? W : tiles);
   uint8_t* d = (uint8_t*)(to_tiles ? tiles : W);
   switch (type) {
-#define C(T) case T: launch_repack_t<T>(to_tiles, wide, grid, st, s, d, stride, n, nb); return GQK_OK;
+#define C(T) case T: launch_repack_t<T>(to_tiles, wide, chunks, st, s, d, stride, n, nb); return GQK_OK;
     C(GQK_Q4_0) C(GQK_Q5_0) C(GQK_Q8_0) C(GQK_Q2_K) C(GQK_Q3_K) C(GQK_Q4_K) C(GQK_Q5_K) C(GQK_Q6_K)
     C(GQK_IQ4_NL) C(GQK_IQ3_S) C(GQK_IQ4_XS)
 #undef C
