@@ -18,6 +18,7 @@ import ctypes
 from dataclasses import dataclass, field
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import GqkPlanInfo, GqkShard, check, lib
@@ -84,8 +85,9 @@ def quant_shape(weight_type: int, n: int, row_bytes: int) -> tuple[int, int]:
     return n, row_bytes // bb * bw
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    """The device's current stream as a raw handle (no Stream object is made)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_gpu(t: torch.Tensor, what: str) -> None:
@@ -314,11 +316,9 @@ def _grouped_into(x: torch.Tensor, packed: torch.Tensor, descs: list[torch.Tenso
         return
     i = _pick_plan(plans, M)
     info = GqkPlanInfo.from_tuple(plans[i * _NPLAN:(i + 1) * _NPLAN])
-    check(lib.gqk_linear(ctypes.c_void_p(packed.data_ptr()), ctypes.c_void_p(descs[i].data_ptr()), ctypes.byref(info),
-                         ctypes.c_void_p(x.data_ptr()), x.stride(0), M, ctypes.c_void_p(out.data_ptr()), out.stride(0),
-                         ctypes.c_void_p(bias.data_ptr() if bias is not None else None),
-                         ctypes.c_void_p(workspace.data_ptr()), workspace.numel() * workspace.element_size(),
-                         _stream(x.device)),
+    check(lib.gqk_linear(packed.data_ptr(), descs[i].data_ptr(), ctypes.byref(info), x.data_ptr(), x.stride(0), M,
+                         out.data_ptr(), out.stride(0), bias.data_ptr() if bias is not None else None,
+                         workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream(x.device)),
           "fused_mul_mat_gguf_grouped")
 
 
@@ -349,6 +349,25 @@ def fused_mul_mat_gguf_grouped_out(x: torch.Tensor, packed: torch.Tensor, descs:
     """As fused_mul_mat_gguf_grouped, writing into `out` (bf16 [M, n_total], unit column stride:
     e.g. the column slice of a wider layer output that this run's shards own)."""
     _grouped_into(x, packed, descs, plans, workspace, bias, out)
+
+
+def _direct(*tensors: torch.Tensor | None) -> bool:
+    """Whether an eager call may go to the library without the dispatcher: nothing traces, transforms
+    or intercepts it (compile, fx and jit tracing, dispatch and function modes, functorch, forward-mode
+    AD) and no tensor needs more than its data pointer (subclasses, lazy negation, autograd).  The
+    dispatcher's share of a custom op call with its two list arguments is about 30 us, several times
+    the launch of a small layer (8 us of GPU time for a 4096 x 4096 Q8_0 layer at one row, whose
+    eager call took 46 us)."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
+            or forward_ad._current_level >= 0):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.is_neg()
+                              or (grad and t.requires_grad)):
+            return False
+    return True
 
 
 def mul_mat_grouped(x: torch.Tensor, gl: GroupedLayer, bias: torch.Tensor | None = None,
@@ -384,6 +403,8 @@ def mul_mat_grouped(x: torch.Tensor, gl: GroupedLayer, bias: torch.Tensor | None
         if xb.shape[0] >= DEQUANT_MIN_M:
             _dequant_mm_into(xb, gl, out)
             fused = None
+        elif _direct(xb, gl.packed, ws, out, fused):
+            _grouped_into(xb, gl.packed, gl.descs, gl.plans, ws, fused, out)
         else:
             fused_mul_mat_gguf_grouped_out(xb, gl.packed, gl.descs, gl.plans, ws, out, fused)
         if bias is not None and fused is None:
@@ -393,6 +414,8 @@ def mul_mat_grouped(x: torch.Tensor, gl: GroupedLayer, bias: torch.Tensor | None
         y = torch.empty((xb.shape[0], gl.n_total), dtype=torch.bfloat16, device=x.device)
         _dequant_mm_into(xb, gl, y)
         fused = None
+    elif _direct(xb, gl.packed, ws, fused):
+        y = _grouped_impl(xb, gl.packed, gl.descs, gl.plans, gl.n_total, ws, fused)
     else:
         y = fused_mul_mat_gguf_grouped(xb, gl.packed, gl.descs, gl.plans, gl.n_total, ws, fused)
     y = y if x.dtype == torch.bfloat16 else y.to(x.dtype)
