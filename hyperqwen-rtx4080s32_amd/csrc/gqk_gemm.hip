@@ -60,12 +60,6 @@ struct Geo {
   static_assert(LDSX + 6160 <= 163840, "LDS");
 };
 
-// a value the whole wave shares, in scalar registers
-__device__ __forceinline__ int64_t g_uniform(int64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
 // One wave's share of a tile: block rb (32 rows) of descriptor row dsc, tokens m0 .. m0 + 32 MB - 1,
 // super-blocks [b0, b1) split over the k-groups.  x comes by buffer loads, not global ones: the
 // compiler counts a global direct-to-LDS load as a flat access and drains every load before the next

@@ -24,8 +24,6 @@ static int64_t stream_k_workgroups(int G, int64_t R, int nb) {
   return std::max<int64_t>(1, std::min<int64_t>({(int64_t)G, R * nb / 4, 6 * R}));
 }
 
-constexpr int64_t kMaxLdx = (int64_t)1 << 22;   // 255 rows of 2 ldx bytes stay below 2^31
-
 static int64_t slot_bytes(int mb, int nr, int wk) { return (int64_t)((4 * mb + wk - 1) / wk) * 64 * nr * wk * 16; }
 
 // The launch of a layer of n_desc descriptor rows at M rows: every geometry's time is estimated from its
@@ -106,7 +104,7 @@ int launch_gemm(const uint8_t* packed, const int32_t* desc, int n_desc, int type
   if ((int64_t)cus * 4 > ctr_bytes || (ctr_bytes & 255)) return GQK_ERR_FORM;
   // A tile's x rows are reached by 32-bit byte offsets from its first one.  Rows further apart than
   // that allows (a view with a row stride above 8 MiB) go one by one, unsplit.
-  if (ldx > kMaxLdx) {
+  if (ldx > GQK_MAX_LDX) {
     GemmPick p = pick(bm, n_desc, 1, nb, cus);
     p.mb = 2, p.nr = 2, p.wk = 4, p.S = 1, p.slots = 0;
     p.grid = (n_desc * p.per + p.nr - 1) / p.nr;

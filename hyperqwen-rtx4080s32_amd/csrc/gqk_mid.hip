@@ -22,7 +22,12 @@ namespace gqk {
 // M = 32: 0.87 / 0.86 / 0.84 / 0.76 of its time; Q2_K, Q8_0, Q6_K down 0.80 / 0.77 / 0.86,
 // IQ4_XS gate_up 0.94; Q6_K and Q8_0 gate_up 1.04).  Tried: weights two steps ahead (more
 // registers, fewer waves: 0-8% slower) and 64 tokens per wave (226-260 VGPRs: 23-45% slower than
-// the 64 x 128 GEMM form, which keeps 33..64 rows).
+// a GEMM form with 64-token tiles).  x and the weights come by buffer loads (a scalar base and one lane
+// offset each, no address arithmetic) and the k-loop is unrolled over a super-block; us at 32 rows
+// before -> now, gate_up / down / qkv / o_proj: Q4_K 38.8 -> 37.8, 25.6 -> 25.3, 12.1 -> 11.2, 11.2 ->
+// 10.4; Q5_K 45.7 -> 42.1, 29.1 -> 27.9, 15.4 -> 14.4, 12.4 -> 11.1; IQ4_XS 40.7 -> 38.0, 29.1 -> 25.6,
+// 13.7 -> 11.9, 13.2 -> 11.4; Q3_K 40.2 -> 34.9, 28.2 -> 24.6, 13.3 -> 11.0, 12.9 -> 10.8; a Q5_K +
+// IQ4_XS layer 49.4 -> 40.5, 33.2 -> 26.9.
 template <int T, int NRB = 2>
 __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, const uint16_t* __restrict__ x, int64_t ldx,
                                          int M, uint16_t* xl, int kw0, int kw1, int c, int r, const GTabs& tb,
@@ -31,30 +36,38 @@ __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, cons
   if (kw0 >= kw1) return;
   // k offsets (within a 64-weight step) of the lane's four 8-weight chunks, in MFMA order
   const int koff[4] = {B2<T>::off0(c), B2<T>::off0(c) + 8, B2<T>::off1(c), B2<T>::off1(c) + 8};
-  const int s0 = 4 * kw0, last = 4 * kw1 - 1;
   // x of a step (32 tokens x 64 k = 32 rows of 128 bytes) comes in with coalesced loads: load i
   // of lane j takes row 8 i + j / 8, 16-byte chunk (j % 8) ^ swz(row), and the wave writes the four
   // loads to its LDS region in lane order; the A operand (token l % 32, chunk koff / 8) is then read
   // at slot chunk ^ swz(token).  swz(t) = (t >> 1) & 7 puts the 16 rows a quarter-wave reads in 16
   // distinct 16-byte bank groups.
   const int lane = threadIdx.x & 63;
-  const uint16_t* xsrc[4];
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, 0xFFFFFFFFu, GQK_GB_WORD3);
+  uint32_t xoff[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = 8 * i + (lane >> 3);
-    xsrc[i] = x + (int64_t)min(t, M - 1) * ldx + 8 * ((lane & 7) ^ ((t >> 1) & 7));
+    xoff[i] = (uint32_t)min(t, M - 1) * (uint32_t)(2 * ldx) + 16u * ((lane & 7) ^ ((t >> 1) & 7));
   }
   const int rs = (r >> 1) & 7;
+  // The two widest types in the slab keep plain weight loads (us at 32 rows, buffer -> plain: Q8_0 qkv /
+  // o_proj 17.4 / 16.0 -> 16.4 / 14.9, Q6_K 16.2 / 14.8 -> 15.6 / 13.8; the others gain by the buffer's),
+  // and Q8_0 in the 64-row form for both (gate_up / down at 20 rows 46.6 / 30.2 -> 45.4 / 29.9).
+  constexpr bool WPTR = T == GQK_Q8_0 || NRB == 1 && T == GQK_Q6_K, XPTR = T == GQK_Q8_0 && NRB == 2;
   struct Step { B2<T> w[NRB]; v4u xg[4]; };
   Step p0, p1;
-  auto load = [&](Step& p, int s) __attribute__((always_inline)) {
+  auto load = [&](Step& p, int kb, int kq) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) p.xg[i] = *(const v4u*)(xsrc[i] + (int64_t)s * 64);
-    const uint8_t* rc = tbase + (int64_t)(s >> 2) * (64 * REC);
+    for (int i = 0; i < 4; ++i)
+      if constexpr (XPTR) p.xg[i] = *(const v4u*)((const uint8_t*)x + xoff[i] + (int64_t)(4 * kb + kq) * (2 * GB_K));
+      else p.xg[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[i], (4 * kb + kq) * (2 * GB_K), 0);
+    const uint8_t* rp = tbase + (int64_t)kb * (64 * REC);
 #pragma unroll
-    for (int b = 0; b < NRB; ++b) p.w[b].load(rc, r0 + 32 * b + r, s & 3, c);
+    for (int b = 0; b < NRB; ++b)
+      if constexpr (WPTR) p.w[b].load(rp, r0 + 32 * b + r, kq, c);
+      else p.w[b].load(g_src(rp), r0 + 32 * b + r, kq, c);
   };
-  auto compute = [&](const Step& p, int s) __attribute__((always_inline)) {
+  auto compute = [&](const Step& p, int kq) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) ((v4u*)xl)[64 * i + lane] = p.xg[i];
     v8bf a[4];
@@ -62,36 +75,60 @@ __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, cons
     for (int q = 0; q < 4; ++q) a[q] = *(const v8bf*)(xl + (r * 8 + ((koff[q] >> 3) ^ rs)) * 8);
 #pragma unroll
     for (int b = 0; b < NRB; ++b) {
-      const GS st = p.w[b].prep(s & 3, c);
+      const GS st = p.w[b].prep(kq, c);
       uint32_t o[16];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p.w[b].out(st, s & 3, c, o, tb, i);
+      for (int i = 0; i < 4; ++i) p.w[b].out(st, kq, c, o, tb, i);
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
             a[q], __builtin_bit_cast(v8bf, v4u{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]}), acc[b], 0, 0, 0);
     }
   };
-  // loads are unconditional (clamped to the wave's last step, re-read from L2 at the tail)
-  load(p0, s0);
-  load(p1, min(s0 + 1, last));
-  for (int s = s0;; s += 2) {
-    compute(p0, s);
-    load(p0, min(s + 2, last));
-    if (s + 1 > last) break;
-    compute(p1, s + 1);
-    load(p1, min(s + 3, last));
-    if (s + 2 > last) break;
+  // Loads are unconditional (clamped to the wave's end, re-read from L2 at the tail).  A super-block's
+  // four steps per trip, so the decoders' shifts and branches on the step fold away, with the next
+  // loads held where they are written (without that the compiler hoists them and takes two waves per
+  // SIMD); Q8_0's decode does not depend on the step and two steps a trip measured 3% faster.
+  if constexpr (T == GQK_Q8_0) {
+    const int last = 4 * kw1 - 1;
+    load(p0, kw0, 0);
+    load(p1, kw0, 1);
+    for (int s = 4 * kw0;; s += 2) {
+      const int s2 = min(s + 2, last), s3 = min(s + 3, last);
+      compute(p0, s & 3);
+      load(p0, s2 >> 2, s2 & 3);
+      if (s + 1 > last) break;
+      compute(p1, (s + 1) & 3);
+      load(p1, s3 >> 2, s3 & 3);
+      if (s + 2 > last) break;
+    }
+    return;
+  }
+  load(p0, kw0, 0);
+  load(p1, kw0, 1);
+  for (int kb = kw0; kb < kw1; ++kb) {
+    const int kn = min(kb + 1, kw1 - 1);
+    compute(p0, 0);
+    load(p0, kb, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(p1, 1);
+    load(p1, kb, 3);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(p0, 2);
+    load(p0, kn, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(p1, 3);
+    load(p1, kn, 1);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 #define MID_RED_BYTES (3 * 2 * 16 * 64 * 4 + 16)   // the waves' sums combined in LDS (nw <= 4), a flag
 
-// Three waves per SIMD for the two instances that would otherwise take just over 168 VGPRs (Q3_K
-// 170, the mixed-type build 176): Q3_K gate_up at M = 20 / 32 2.0-2.9 us faster; mixed layers
-// (gate_up, qkv + o_proj) 0.5-2.4 us faster even with the mixed build's 20 bytes of scratch.
+// Three waves per SIMD: every type fits 168 VGPRs without scratch (151-168); Q8_0 has its loads placed
+// as well as two waves' registers allow instead (above).
 template <int ONLY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK_Q3_K || ONLY == 0 ? 3 : 1))) void gemv_mid_kernel(const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK_Q8_0 ? 1 : 3))) void gemv_mid_kernel(const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc,
                                                        const uint16_t* __restrict__ x, int64_t ldx, int M,
                                                        uint16_t* __restrict__ y, int64_t ldy,
                                                        const uint16_t* __restrict__ bias, float* __restrict__ part,
@@ -136,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK
     for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
 #define RUN(T)                                                                                                 \
   if ((ONLY == 0 || ONLY == T) && type == T)                                                                   \
-    mid_wave<T>(packed + off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC), x, ldx, M, xl, kw0, kw1, c, r, tb, acc);
+    mid_wave<T>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, acc);
   RUN(GQK_Q4_0) RUN(GQK_Q5_0) RUN(GQK_Q8_0) RUN(GQK_Q2_K) RUN(GQK_Q3_K) RUN(GQK_Q4_K) RUN(GQK_Q5_K) RUN(GQK_Q6_K)
   RUN(GQK_IQ4_NL) RUN(GQK_IQ3_S) RUN(GQK_IQ4_XS)
 #undef RUN
@@ -288,7 +325,7 @@ __global__ __launch_bounds__(64 * GQK_SLAB_MAX_WAVES) void gemv_mid_slab_kernel(
   for (int v = 0; v < 16; ++v) acc[0][v] = 0.f;
 #define RUN(T)                                                                                                 \
   if ((ONLY == 0 || ONLY == T) && type == T)                                                                   \
-    mid_wave<T, 1>(packed + off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC), x, ldx, M, xl, kw0, kw1, c, r, tb, \
+    mid_wave<T, 1>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, \
                    acc, 32 * h);
   RUN(GQK_Q4_0) RUN(GQK_Q5_0) RUN(GQK_Q8_0) RUN(GQK_Q2_K) RUN(GQK_Q3_K) RUN(GQK_Q4_K) RUN(GQK_Q5_K) RUN(GQK_Q6_K)
   RUN(GQK_IQ4_NL) RUN(GQK_IQ3_S) RUN(GQK_IQ4_XS)

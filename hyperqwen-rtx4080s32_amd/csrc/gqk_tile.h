@@ -50,6 +50,12 @@ __device__ __forceinline__ void gld(uint32_t* dst, const uint8_t* p) {
   }
 }
 
+// a value the whole wave shares, in scalar registers
+__device__ __forceinline__ int64_t g_uniform(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // A byte address with a part the whole wave shares (scalar base, scalar offset) and a lane's 32-bit
 // offset: one buffer load, no address arithmetic in vector registers.  c + n moves the shared part,
 // c[n] adds a lane offset.

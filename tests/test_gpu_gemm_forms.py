@@ -58,13 +58,14 @@ def test_geometries(dev, shards, nbk):
 
 
 def test_rows_far_apart(dev):
-    """A row stride above 8 MiB: the rows go one by one."""
+    """A row stride above 8 MiB: the rows of the mid form and the GEMM go one by one."""
     import gguf_hip
 
-    K, M, ldx = 512, 34, (1 << 22) + 64
+    K, ldx = 512, (1 << 22) + 64
     gl, wf = _layer(dev, [(G.Q4_K, 130)], K, 3)
-    buf = torch.zeros((M - 1) * ldx + K, dtype=torch.bfloat16, device=dev)
-    x = buf.as_strided((M, K), (ldx, 1))
-    x.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16))
-    y = gguf_hip.mul_mat_grouped(x, gl)
-    assert _close(y.float().cpu().numpy(), x.float().cpu().numpy(), wf)
+    buf = torch.zeros(33 * ldx + K, dtype=torch.bfloat16, device=dev)
+    for M in (3, 18, 34):
+        x = buf.as_strided((M, K), (ldx, 1))
+        x.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16))
+        y = gguf_hip.mul_mat_grouped(x, gl)
+        assert _close(y.float().cpu().numpy(), x.float().cpu().numpy(), wf), M
