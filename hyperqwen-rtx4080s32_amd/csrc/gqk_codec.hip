@@ -83,9 +83,14 @@ __device__ __forceinline__ void decode(const S& s, int i, const uint32_t* grid, 
   constexpr bool MIN = T == GQK_Q2_K || T == GQK_Q4_K || T == GQK_Q5_K;
   uint2 q;
   uint32_t qn[N / 4];   // the N integers
+  // N == 4: the half by arithmetic.  i & 1 ? q.y : q.x became an indexed load of q kept in memory (LDS),
+  // whose address takes the workgroup size from the dispatch packet, a read of host memory: Q4_K to
+  // fp32 from rows, us with that -> so: 4096 x 512 19.2 -> 5.4, 4096 x 4096 29.2 -> 16.3, 17408 x 5120
+  // 137 -> 105 (with 32 weights a thread 6.6, 27.9, 145).
   auto narrow = [&] {
-    if constexpr (N == 8) qn[0] = q.x, qn[1] = q.y;
-    else qn[0] = i & 1 ? q.y : q.x;
+    const uint32_t lo = q.x, hi = q.y;
+    if constexpr (N == 8) qn[0] = lo, qn[1] = hi;
+    else qn[0] = lo ^ ((lo ^ hi) & -(uint32_t)(i & 1));
   };
   if constexpr (T == GQK_Q4_0 || T == GQK_IQ4_NL || T == GQK_Q5_0) {   // low nibbles: weights 0..15, high: 16..31
     constexpr int PD = T == GQK_Q5_0 ? 2 : 1;
