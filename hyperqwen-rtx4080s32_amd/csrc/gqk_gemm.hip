@@ -194,8 +194,9 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ packed, co
   for (int i = 0; i < MB; ++i) A[i] = aread(xq[0], i);
   int it = 0;
   // Before step s' barrier a wave's part of x(s + 1) is in LDS: after its loads (two steps ago) the
-  // wave issued x(s + 2) and two steps' weights, at least one load each, so x(s + 1) is complete when
-  // at most XI + 2 loads are outstanding (memory operations complete in order).
+  // wave issued x(s + 2) and two steps' weights, so x(s + 1) is complete when at most XI + 2 loads are
+  // outstanding (memory operations complete in order).  At the second step only the first one's weights
+  // follow x(s + 1): the count needs two weight loads a step, which every decoder issues.
   for (int sb = g0; sb < g1; ++sb, ++it) {
     step(std::integral_constant<int, 0>{}, sb, w0, w1, w3);
     step(std::integral_constant<int, 1>{}, sb, w1, w2, w0);

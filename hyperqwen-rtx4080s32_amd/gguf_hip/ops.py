@@ -354,7 +354,8 @@ def fused_mul_mat_gguf_grouped_out(x: torch.Tensor, packed: torch.Tensor, descs:
 def _direct(*tensors: torch.Tensor | None) -> bool:
     """Whether an eager call may go to the library without the dispatcher: nothing traces, transforms
     or intercepts it (compile, fx and jit tracing, dispatch and function modes, functorch, forward-mode
-    AD) and no tensor needs more than its data pointer (subclasses, lazy negation, autograd).  The
+    AD) and no tensor needs more than its data pointer (subclasses, lazy negation, functional and zero
+    tensors, autograd).  The
     dispatcher's share of a custom op call with its two list arguments is about 30 us, several times
     the launch of a small layer (8 us of GPU time for a 4096 x 4096 Q8_0 layer at one row, whose
     eager call took 46 us)."""
@@ -365,7 +366,7 @@ def _direct(*tensors: torch.Tensor | None) -> bool:
     grad = torch.is_grad_enabled()
     for t in tensors:
         if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.is_neg()
-                              or (grad and t.requires_grad)):
+                              or t._is_zerotensor() or torch._is_functional_tensor(t) or (grad and t.requires_grad)):
             return False
     return True
 
@@ -405,6 +406,8 @@ def mul_mat_grouped(x: torch.Tensor, gl: GroupedLayer, bias: torch.Tensor | None
             fused = None
         elif _direct(xb, gl.packed, ws, out, fused):
             _grouped_into(xb, gl.packed, gl.descs, gl.plans, ws, fused, out)
+            # as the op does: autograd then refuses a graph that had saved out's old values
+            torch.autograd.graph.increment_version(out)
         else:
             fused_mul_mat_gguf_grouped_out(xb, gl.packed, gl.descs, gl.plans, ws, out, fused)
         if bias is not None and fused is None:

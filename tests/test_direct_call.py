@@ -25,6 +25,8 @@ def test_direct_only_for_plain_eager_tensors():
         assert _direct(torch.randn(2))
     assert not _direct(x.as_subclass(_Sub))
     assert not _direct(torch._neg_view(x))
+    assert not _direct(torch._efficientzerotensor((3,)))
+    assert not _direct(torch._to_functional_tensor(x))
     mode = FakeTensorMode()
     with mode:
         assert not _direct(x)
@@ -42,6 +44,23 @@ def test_direct_only_for_plain_eager_tensors():
     torch.func.functionalize(lambda t: (seen.append(_direct(x)), t)[1])(x)
     torch.jit.trace(lambda t: (seen.append(_direct(t)), t + 1)[1], (x,), check_trace=False)
     assert seen and not any(seen), seen
+
+
+def test_direct_write_bumps_the_output_version(monkeypatch):
+    import types
+
+    from gguf_hip import ops
+
+    monkeypatch.setattr(ops, "_require_gpu", lambda t, what: None)
+    monkeypatch.setattr(ops, "_grouped_into", lambda *a: None)   # the library writes past torch
+    gl = types.SimpleNamespace(K=256, n_total=64, packed=torch.zeros(8, dtype=torch.uint8), descs=[], plans=[],
+                               workspace=torch.zeros(8, dtype=torch.int32))
+    x, out = (torch.ones(4, k, dtype=torch.bfloat16) for k in (256, 64))
+    w = torch.ones(4, 64, dtype=torch.bfloat16, requires_grad=True)
+    loss = (w * out).sum()   # saves out
+    ops.mul_mat_grouped(x, gl, out=out)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
 
 
 @pytest.mark.gpu
