@@ -39,6 +39,7 @@ def _layer(dev, shards, K, seed):
     ([(G.IQ4_XS, 640), (G.Q2_K, 70), (G.Q5_0, 129)], 7),
     ([(G.Q5_K, 2100)], 9),
     ([(G.IQ4_NL, 33), (G.Q4_0, 64)], 13),
+    ([(G.Q4_K, 1097)], 4),                                  # unsplit: eights of tiles and a rest, dealt to XCDs
 ])
 def test_geometries(dev, shards, nbk):
     import gguf_hip
