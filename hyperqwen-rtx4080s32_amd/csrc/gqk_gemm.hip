@@ -348,7 +348,12 @@ __global__ __launch_bounds__(GE::NT) __attribute__((amdgpu_waves_per_eu(GE::WPE)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nmb = (M + GE::BM - 1) / GE::BM;
   const int nb = __builtin_amdgcn_readfirstlane(desc[D_NB]);
-  auto run = [&](int tile, int mb, int b0, int b1, const GOut& go) {
+  // Inlined by force: in the mixed-type 256 x 256 build the compiler left it out of line, where its code
+  // is longer than a branch reaches and the long branches overwrote the return address (the kernel never
+  // ended), and its uniform operands came back from the stack as vector values.  us, the form before the
+  // register decode (out of line too) -> this: Q4_K + Q6_K 7168 x 5120 at 768 / 2048 rows 164 -> 89, 298 ->
+  // 165; Q5_K + IQ4_XS 34816 x 5120 at 512 / 2048 409 -> 208, 1347 -> 685.
+  auto run = [&](int tile, int mb, int b0, int b1, const GOut& go) __attribute__((always_inline)) {
     tile = __builtin_amdgcn_readfirstlane(tile);
     mb = __builtin_amdgcn_readfirstlane(mb);
     b0 = __builtin_amdgcn_readfirstlane(b0);
