@@ -518,14 +518,9 @@ int gqk_linear(const void* packed, const int32_t* desc_dev, const gqk_plan_info*
       counters = (int*)workspace;
       partials = (float*)((char*)workspace + cb);
     }
-    // the mid form reaches x rows by 32-bit byte offsets from the first: rows further apart go one by one
-    const int step = info->g == 8 && ldx > GQK_MAX_LDX ? 1 : M;
-    for (int t = 0; t < M; t += step) {
-      int rc = gqk::launch_gemv((const uint8_t*)packed, desc_dev, info->n_desc, info->types_mask,
-                                (const uint16_t*)x + t * ldx, ldx, step, info->g, info->nw, info->bm, info->nb,
-                                (uint16_t*)y + t * ldy, ldy, bias, partials, counters, (hipStream_t)stream);
-      if (rc) return fail(rc, "linear: GEMV launch form");
-    }
+    int rc = gqk::launch_gemv((const uint8_t*)packed, desc_dev, info->n_desc, info->types_mask, x, ldx, M, info->g, info->nw,
+                              info->bm, info->nb, y, ldy, bias, partials, counters, (hipStream_t)stream);
+    if (rc) return fail(rc, "linear: GEMV launch form");
     return check_launch("linear (GEMV)");
   }
   if (info->form == GQK_FORM_GEMM) {

@@ -137,7 +137,8 @@ GQK_LAYOUT(GQK_IQ4_XS, 136, 0, 128)
 // device serves all layers and batch sizes: no plan's fp32 partials overlap another's counters.
 #define GQK_CTR_BYTES 262144   // (mirrored in include/gguf_hip.h)
 #define GQK_CTR_WORDS (GQK_CTR_BYTES / 4)
-#define GQK_MAX_LDX (1 << 22)   // row stride of x up to which 255 rows of 2 ldx bytes stay below 2^31
+#define GQK_MAX_LDX (1 << 22)   // row stride of x up to which 255 rows of 2 ldx bytes stay below 2^31; above it
+                                // the GEMM and the mid form launch their builds with 64-bit row addresses
 #define GQK_GEMV_MAX_M 32   // batch rows of the streaming forms (GEMV up to 16, mid form 17..32); GEMM above
 #define GQK_GEMV_MAX_WAVES 8   // waves per GEMV workgroup (two per SIMD: no register bound below 256)
 #define GQK_GEMV_SLAB 2        // plan bm of the GEMV slab form (M <= 8: a workgroup per 32-row slab, x in LDS)

@@ -64,8 +64,10 @@ struct Geo {
 // super-blocks [b0, b1) split over the k-groups.  x comes by buffer loads, not global ones: the
 // compiler counts a global direct-to-LDS load as a flat access and drains every load before the next
 // LDS read (measured: 684 -> 655 us at 2048 rows); the weights too (scalar base + one lane offset: no
-// address registers).
-template <class GE, int T>
+// address registers).  FAR: rows of x further apart than 32-bit byte offsets from the tile's first one
+// reach (GQK_MAX_LDX) come by global loads from a 64-bit address each (Q4_K 5120 x 5120 at 64 / 128 rows
+// 20 MiB apart 15.3 / 23.1 us; near rows 14.6 / 19.6, a launch per row 1054 / 2105).
+template <class GE, int T, bool FAR>
 __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ packed, const int32_t* __restrict__ dsc,
                                         int rb, const uint16_t* __restrict__ x, int64_t ldx, int M, int m0, int b0, int b1,
                                         const GOut& go, uint16_t* __restrict__ y, int64_t ldy,
@@ -81,11 +83,11 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ packed, co
   const uint8_t* wb = packed + g_uniform(off + (tile0 + (btile < ntiles ? btile : 0)) * nb * (int64_t)(64 * REC));
   const __amdgpu_buffer_rsrc_t xr =
       __builtin_amdgcn_make_buffer_rsrc((void*)(x + (int64_t)m0 * ldx), 0, 0xFFFFFFFFu, GQK_GB_WORD3);
-  uint32_t xoff[XI];
+  std::conditional_t<FAR, int64_t, uint32_t> xoff[XI];
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
     const int row = 8 * min(wr + NR * i, GE::XN - 1) + (lane >> 3);
-    xoff[i] = (uint32_t)min(row, M - 1 - m0) * (uint32_t)(2 * ldx) + 16u * ((lane & 7) ^ ((row >> 1) & 7));
+    xoff[i] = min(row, M - 1 - m0) * (decltype(+xoff[i]))(2 * ldx) + 16u * ((lane & 7) ^ ((row >> 1) & 7));
   }
   uint16_t* xs = xlds + wg * (GE::D * GE::STG);
   const int koff[4] = {B2<T>::off0(h), B2<T>::off0(h) + 8, B2<T>::off1(h), B2<T>::off1(h) + 8};
@@ -108,10 +110,15 @@ __device__ __forceinline__ void gemm_tile(const uint8_t* __restrict__ packed, co
   auto dma = [&](int buf, int s) __attribute__((always_inline)) {
 #ifdef __HIP_DEVICE_COMPILE__   // the host pass rejects 16-byte direct-to-LDS loads
 #pragma unroll
-    for (int i = 0; i < XI; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          xr, (__attribute__((address_space(3))) void*)(xs + buf * GE::STG + 512 * min(wr + NR * i, GE::XN - 1)), 16, xoff[i],
-          s * (2 * GB_K), 0, 0);
+    for (int i = 0; i < XI; ++i) {
+      const auto to = (__attribute__((address_space(3))) void*)(xs + buf * GE::STG + 512 * min(wr + NR * i, GE::XN - 1));
+      if constexpr (FAR)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)((const uint8_t*)(x + (int64_t)m0 * ldx) + xoff[i] + (int64_t)s * (2 * GB_K)),
+            to, 16, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, xoff[i], s * (2 * GB_K), 0, 0);
+    }
 #endif
   };
   auto aread = [&](lptr b, int i) __attribute__((always_inline)) {
@@ -334,7 +341,8 @@ __device__ __forceinline__ void gb_map(int i, int n_desc, int nmb, int& d, int& 
 // floor(T / G) * G tiles whole, dealt round robin; the remaining R tiles' super-blocks split evenly over
 // gsk workgroups (stream-K), shared tiles combined the same way.  The waves of a workgroup may hold
 // blocks of different shards and types: every type's code meets the same barriers.
-template <class GE, int ONLY>
+// FAR: the mixed-type build (ONLY = 0) serves every layer.
+template <class GE, int ONLY, bool FAR = false>
 __global__ __launch_bounds__(GE::NT) __attribute__((amdgpu_waves_per_eu(GE::WPE))) void gemm_kernel(
     const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc, int n_desc, const uint16_t* __restrict__ x,
     int64_t ldx, int M, uint16_t* __restrict__ y, int64_t ldy, const uint16_t* __restrict__ bias, float* part, int* ctr,
@@ -365,7 +373,7 @@ __global__ __launch_bounds__(GE::NT) __attribute__((amdgpu_waves_per_eu(GE::WPE)
     const int type = __builtin_amdgcn_readfirstlane(dsc[D_TYPE]);
 #define RUN(TY)                                                                                          \
     if ((ONLY == 0 || ONLY == TY) && type == TY)                                                         \
-      gemm_tile<GE, TY>(packed, dsc, rb, x, ldx, M, mb * GE::BM, b0, b1, go, y, ldy, bias, xs, flag, tb);
+      gemm_tile<GE, TY, FAR>(packed, dsc, rb, x, ldx, M, mb * GE::BM, b0, b1, go, y, ldy, bias, xs, flag, tb);
     RUN(GQK_Q4_0) RUN(GQK_Q5_0) RUN(GQK_Q8_0) RUN(GQK_Q2_K) RUN(GQK_Q3_K) RUN(GQK_Q4_K) RUN(GQK_Q5_K) RUN(GQK_Q6_K)
     RUN(GQK_IQ4_NL) RUN(GQK_IQ3_S) RUN(GQK_IQ4_XS)
 #undef RUN
@@ -434,6 +442,10 @@ static int launch_geo(const GemmPick& p, int only, int n_desc, int M, hipStream_
                       const int32_t* desc, const uint16_t* x, int64_t ldx, uint16_t* y, int64_t ldy,
                       const uint16_t* bias, float* part, int* ctr) {
   const dim3 grid(p.grid), block(GE::NT);
+  if (ldx > GQK_MAX_LDX) {
+    hipLaunchKernelGGL((gemm_kernel<GE, 0, true>), grid, block, 0, st, packed, desc, n_desc, x, ldx, M, y, ldy, bias, part, ctr, p.per, p.G, p.gsk, p.S);
+    return GQK_OK;
+  }
   switch (only) {
 #define C(T) case T: hipLaunchKernelGGL((gemm_kernel<GE, T>), grid, block, 0, st, packed, desc, n_desc, x, ldx, M, y, ldy, bias, part, ctr, p.per, p.G, p.gsk, p.S); return GQK_OK;
     C(GQK_Q4_0) C(GQK_Q5_0) C(GQK_Q8_0) C(GQK_Q2_K) C(GQK_Q3_K) C(GQK_Q4_K) C(GQK_Q5_K) C(GQK_Q6_K)

@@ -102,19 +102,6 @@ int launch_gemm(const uint8_t* packed, const int32_t* desc, int n_desc, int type
   const int nb = (int)(K / 256), cus = gb_cus();
   if (cus <= 0) return GQK_ERR_HIP;
   if ((int64_t)cus * 4 > ctr_bytes || (ctr_bytes & 255)) return GQK_ERR_FORM;
-  // A tile's x rows are reached by 32-bit byte offsets from its first one.  Rows further apart than
-  // that allows (a view with a row stride above 8 MiB) go one by one, unsplit.
-  if (ldx > GQK_MAX_LDX) {
-    GemmPick p = pick(bm, n_desc, 1, nb, cus);
-    p.mb = 2, p.nr = 2, p.wk = 4, p.S = 1, p.slots = 0;
-    p.grid = (n_desc * p.per + p.nr - 1) / p.nr;
-    for (int t = 0; t < M; ++t) {
-      const int rc = launch_gemm_mb2(p, types_mask, n_desc, 1, st, packed, desc, (const uint16_t*)x + t * ldx, ldx,
-                                     (uint16_t*)y + t * ldy, ldy, (const uint16_t*)bias, nullptr, nullptr);
-      if (rc) return rc;
-    }
-    return GQK_OK;
-  }
   const GemmPick p = pick(bm, n_desc, M, nb, cus);
   const int64_t need = pick_bytes(p, ctr_bytes);
   if (need > 0 && (ws == nullptr || ws_bytes < need || ((uintptr_t)ws & 255))) return GQK_ERR_SHAPE;

@@ -28,7 +28,8 @@ namespace gqk {
 // 10.4; Q5_K 45.7 -> 42.1, 29.1 -> 27.9, 15.4 -> 14.4, 12.4 -> 11.1; IQ4_XS 40.7 -> 38.0, 29.1 -> 25.6,
 // 13.7 -> 11.9, 13.2 -> 11.4; Q3_K 40.2 -> 34.9, 28.2 -> 24.6, 13.3 -> 11.0, 12.9 -> 10.8; a Q5_K +
 // IQ4_XS layer 49.4 -> 40.5, 33.2 -> 26.9.
-template <int T, int NRB = 2>
+// FAR: rows of x further apart than 32-bit byte offsets reach (GQK_MAX_LDX), by 64-bit addresses.
+template <int T, int NRB = 2, bool FAR = false>
 __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, const uint16_t* __restrict__ x, int64_t ldx,
                                          int M, uint16_t* xl, int kw0, int kw1, int c, int r, const GTabs& tb,
                                          v16f (&acc)[NRB], int r0 = 0) {
@@ -43,17 +44,17 @@ __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, cons
   // distinct 16-byte bank groups.
   const int lane = threadIdx.x & 63;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, 0xFFFFFFFFu, GQK_GB_WORD3);
-  uint32_t xoff[4];
+  std::conditional_t<FAR, int64_t, uint32_t> xoff[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = 8 * i + (lane >> 3);
-    xoff[i] = (uint32_t)min(t, M - 1) * (uint32_t)(2 * ldx) + 16u * ((lane & 7) ^ ((t >> 1) & 7));
+    xoff[i] = min(t, M - 1) * (decltype(+xoff[i]))(2 * ldx) + 16u * ((lane & 7) ^ ((t >> 1) & 7));
   }
   const int rs = (r >> 1) & 7;
   // The two widest types in the slab keep plain weight loads (us at 32 rows, buffer -> plain: Q8_0 qkv /
   // o_proj 17.4 / 16.0 -> 16.4 / 14.9, Q6_K 16.2 / 14.8 -> 15.6 / 13.8; the others gain by the buffer's),
   // and Q8_0 in the 64-row form for both (gate_up / down at 20 rows 46.6 / 30.2 -> 45.4 / 29.9).
-  constexpr bool WPTR = T == GQK_Q8_0 || NRB == 1 && T == GQK_Q6_K, XPTR = T == GQK_Q8_0 && NRB == 2;
+  constexpr bool WPTR = T == GQK_Q8_0 || NRB == 1 && T == GQK_Q6_K, XPTR = FAR || T == GQK_Q8_0 && NRB == 2;
   struct Step { B2<T> w[NRB]; v4u xg[4]; };
   Step p0, p1;
   auto load = [&](Step& p, int kb, int kq) __attribute__((always_inline)) {
@@ -127,8 +128,8 @@ __device__ __forceinline__ void mid_wave(const uint8_t* __restrict__ tbase, cons
 
 // Three waves per SIMD: every type fits 168 VGPRs without scratch (151-168); Q8_0 has its loads placed
 // as well as two waves' registers allow instead (above).
-template <int ONLY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK_Q8_0 ? 1 : 3))) void gemv_mid_kernel(const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc,
+template <int ONLY, bool FAR = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK_Q8_0 || FAR ? 1 : 3))) void gemv_mid_kernel(const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc,
                                                        const uint16_t* __restrict__ x, int64_t ldx, int M,
                                                        uint16_t* __restrict__ y, int64_t ldy,
                                                        const uint16_t* __restrict__ bias, float* __restrict__ part,
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK
     for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
 #define RUN(T)                                                                                                 \
   if ((ONLY == 0 || ONLY == T) && type == T)                                                                   \
-    mid_wave<T>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, acc);
+    mid_wave<T, 2, FAR>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, acc);
   RUN(GQK_Q4_0) RUN(GQK_Q5_0) RUN(GQK_Q8_0) RUN(GQK_Q2_K) RUN(GQK_Q3_K) RUN(GQK_Q4_K) RUN(GQK_Q5_K) RUN(GQK_Q6_K)
   RUN(GQK_IQ4_NL) RUN(GQK_IQ3_S) RUN(GQK_IQ4_XS)
 #undef RUN
@@ -285,7 +286,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONLY == GQK
 // rows each; no split-K partials (whose 8 KiB per workgroup at 32 tokens made the exchange ~30% of
 // the mid form's qkv / o_proj launches).  Each wave's sums go to its own 4 KiB x region once its
 // products are done, and after one barrier every thread sums one output over the waves in order.
-template <int ONLY>
+template <int ONLY, bool FAR = false>
 __global__ __launch_bounds__(64 * GQK_SLAB_MAX_WAVES) void gemv_mid_slab_kernel(
     const uint8_t* __restrict__ packed, const int32_t* __restrict__ desc, const uint16_t* __restrict__ x,
     int64_t ldx, int M, uint16_t* __restrict__ y, int64_t ldy, const uint16_t* __restrict__ bias) {
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(64 * GQK_SLAB_MAX_WAVES) void gemv_mid_slab_kernel(
   for (int v = 0; v < 16; ++v) acc[0][v] = 0.f;
 #define RUN(T)                                                                                                 \
   if ((ONLY == 0 || ONLY == T) && type == T)                                                                   \
-    mid_wave<T, 1>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, \
+    mid_wave<T, 1, FAR>(packed + g_uniform(off + tile * nb * (int64_t)(64 * gqk_layout<T>::REC)), x, ldx, M, xl, kw0, kw1, c, r, tb, \
                    acc, 32 * h);
   RUN(GQK_Q4_0) RUN(GQK_Q5_0) RUN(GQK_Q8_0) RUN(GQK_Q2_K) RUN(GQK_Q3_K) RUN(GQK_Q4_K) RUN(GQK_Q5_K) RUN(GQK_Q6_K)
   RUN(GQK_IQ4_NL) RUN(GQK_IQ3_S) RUN(GQK_IQ4_XS)
@@ -357,9 +358,14 @@ int launch_gemv_mid(const uint8_t* packed, const int32_t* desc, int n_desc, int 
   const uint16_t* xx = (const uint16_t*)x;
   uint16_t* yy = (uint16_t*)y;
   const uint16_t* bb = (const uint16_t*)bias;
+  const bool far = ldx > GQK_MAX_LDX;   // the mixed-type builds serve every layer there
   if (slab) {
     if (nw < 1 || nw > GQK_SLAB_MAX_WAVES) return GQK_ERR_FORM;
     const dim3 grid(n_desc), block(64 * nw);
+    if (far) {
+      hipLaunchKernelGGL((gemv_mid_slab_kernel<0, true>), grid, block, 0, st, packed, desc, xx, ldx, M, yy, ldy, bb);
+      return GQK_OK;
+    }
     switch (types_mask) {
 #define C(T) case T: hipLaunchKernelGGL((gemv_mid_slab_kernel<T>), grid, block, 0, st, packed, desc, xx, ldx, M, yy, ldy, bb); return GQK_OK;
       C(GQK_Q4_0) C(GQK_Q5_0) C(GQK_Q8_0) C(GQK_Q2_K) C(GQK_Q3_K) C(GQK_Q4_K) C(GQK_Q5_K) C(GQK_Q6_K)
@@ -372,6 +378,10 @@ int launch_gemv_mid(const uint8_t* packed, const int32_t* desc, int n_desc, int 
   }
   if (nw < 1 || nw > 4) return GQK_ERR_FORM;
   const dim3 grid(n_desc), block(64 * nw);
+  if (far) {
+    hipLaunchKernelGGL((gemv_mid_kernel<0, true>), grid, block, 0, st, packed, desc, xx, ldx, M, yy, ldy, bb, part, ctr);
+    return GQK_OK;
+  }
   switch (types_mask) {
 #define C(T) case T: hipLaunchKernelGGL((gemv_mid_kernel<T>), grid, block, 0, st, packed, desc, xx, ldx, M, yy, ldy, bb, part, ctr); return GQK_OK;
     C(GQK_Q4_0) C(GQK_Q5_0) C(GQK_Q8_0) C(GQK_Q2_K) C(GQK_Q3_K) C(GQK_Q4_K) C(GQK_Q5_K) C(GQK_Q6_K)

@@ -22,14 +22,14 @@ def _close(y, x, wf, bias=None):
         np.linalg.norm(err) <= 1e-2 * np.linalg.norm(ref)
 
 
-def _layer(dev, shards, K, seed):
+def _layer(dev, shards, K, seed, cus=0):
     import gguf_hip
 
     rng = np.random.default_rng(seed)
     raws = [G.make_weights(rng, n, K, wt) for wt, n in shards]
     wf = np.concatenate([G.dequantize(r, wt) for r, (wt, _) in zip(raws, shards)])
     return gguf_hip.pack_layer([torch.from_numpy(r).to(dev) for r in raws], [n for _, n in shards],
-                               [wt for wt, _ in shards]), wf
+                               [wt for wt, _ in shards], cus=cus), wf
 
 
 @pytest.mark.parametrize("shards,nbk", [
@@ -97,15 +97,40 @@ def test_persistent_tiles_of_every_type(dev, n0, nbk, M):
     assert int(gl.workspace[:info.ctr_bytes // 4].abs().sum()) == 0
 
 
-def test_rows_far_apart(dev):
-    """A row stride above 8 MiB: the rows of the mid form and the GEMM go one by one."""
+def _launches(fn):
+    """fn()'s result and how many kernels of the linear forms it launched."""
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        y = fn()
+        torch.cuda.synchronize()
+    return y, sum("gemm_kernel" in e.name or "gemv" in e.name for e in prof.events())
+
+
+@pytest.mark.parametrize("ldx", [1 << 22, (1 << 22) + 8, (1 << 27) + 64])
+def test_rows_far_apart(dev, ldx):
+    """Row strides of x at the last one that 32-bit byte offsets from a tile's first row serve (8 MiB), just
+    above it, and where such offsets would wrap within 32 rows: one launch each, the same bits as from a
+    contiguous x, in the mid form (slab and split), the GEMM (split) and the 256 x 256 form."""
     import gguf_hip
 
-    K, ldx = 512, (1 << 22) + 64
-    gl, wf = _layer(dev, [(G.Q4_K, 130)], K, 3)
-    buf = torch.zeros(33 * ldx + K, dtype=torch.bfloat16, device=dev)
-    for M in (3, 18, 34):
-        x = buf.as_strided((M, K), (ldx, 1))
+    K = 512
+    small, wf = _layer(dev, [(G.Q4_K, 130), (G.IQ3_S, 64)], K, 3)
+    slab, _ = _layer(dev, [(G.Q4_K, 130), (G.IQ3_S, 64)], K, 3, cus=8)
+    wide = None
+    if ldx < 1 << 23:
+        from gguf_hip.synth import random_shard
+
+        ns = [800 + 7 * i for i in range(len(G.ALL_TYPES))]
+        wide = gguf_hip.pack_layer([random_shard(n, K, t, dev, seed=t) for n, t in zip(ns, G.ALL_TYPES)], ns, list(G.ALL_TYPES))
+    for gl, M in ((small, 3), (small, 18), (slab, 32), (small, 34), (small, 41), (wide, 1801)):
+        if gl is None:
+            continue
+        x = torch.empty((M - 1) * ldx + K, dtype=torch.bfloat16, device=dev).as_strided((M, K), (ldx, 1))
         x.copy_(torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16))
-        y = gguf_hip.mul_mat_grouped(x, gl)
-        assert _close(y.float().cpu().numpy(), x.float().cpu().numpy(), wf), M
+        print(ldx, M, flush=True)
+        y, count = _launches(lambda: gguf_hip.mul_mat_grouped(x, gl))
+        assert count == 1, (M, count)
+        assert torch.equal(y, gguf_hip.mul_mat_grouped(x.contiguous(), gl)), M
+        if gl is not wide:
+            assert _close(y.float().cpu().numpy(), x.float().cpu().numpy(), wf), M
+        del x
