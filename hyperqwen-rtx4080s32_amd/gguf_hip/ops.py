@@ -18,7 +18,7 @@ import ctypes
 from dataclasses import dataclass, field
 
 import torch
-from torch.autograd import forward_ad
+from torch.autograd import forward_ad, profiler
 
 from . import _lib
 from ._lib import GqkPlanInfo, GqkShard, check, lib
@@ -354,12 +354,13 @@ def fused_mul_mat_gguf_grouped_out(x: torch.Tensor, packed: torch.Tensor, descs:
 def _direct(*tensors: torch.Tensor | None) -> bool:
     """Whether an eager call may go to the library without the dispatcher: nothing traces, transforms
     or intercepts it (compile, fx and jit tracing, dispatch and function modes, functorch, forward-mode
-    AD) and no tensor needs more than its data pointer (subclasses, lazy negation, functional and zero
-    tensors, autograd).  The
-    dispatcher's share of a custom op call with its two list arguments is about 30 us, several times
-    the launch of a small layer (8 us of GPU time for a 4096 x 4096 Q8_0 layer at one row, whose
-    eager call took 46 us)."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+    AD), no profiler records the ops, and no tensor needs more than its data pointer (subclasses, lazy
+    negation, functional and zero tensors, autograd).  The dispatcher's share of a custom op call with
+    its two list arguments is about 30 us, several times the launch of a small layer (8 us of GPU time
+    for a 4096 x 4096 Q8_0 layer at one row, whose eager call took 46 us).  An ExecutionTraceObserver
+    that runs without a profiler cannot be seen from here: it misses the op."""
+    if (torch.compiler.is_compiling() or profiler._is_profiler_enabled or torch.autograd._profiler_enabled()
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
             or forward_ad._current_level >= 0):
         return False

@@ -63,6 +63,22 @@ def test_direct_write_bumps_the_output_version(monkeypatch):
         loss.backward()
 
 
+def test_a_profiler_sees_the_op():
+    import threading
+
+    from gguf_hip.ops import _direct
+
+    x, seen = torch.randn(4, 8), []
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        seen.append(_direct(x))
+        t = threading.Thread(target=lambda: seen.append(_direct(x)))
+        t.start()
+        t.join()
+    with torch.autograd.profiler.profile():
+        seen.append(_direct(x))
+    assert seen == [False] * 3 and _direct(x)
+
+
 @pytest.mark.gpu
 def test_direct_and_dispatched_calls_agree(dev):
     import gguf_hip
