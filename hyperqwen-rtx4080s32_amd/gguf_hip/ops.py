@@ -18,10 +18,10 @@ import ctypes
 from dataclasses import dataclass, field
 
 import torch
-from torch.autograd import forward_ad, profiler
 
 from . import _lib
 from ._lib import GqkPlanInfo, GqkShard, check, lib
+from .eager import direct as _direct, stream as _stream
 
 # GGML type ids served by the library (ggml.h enum)
 Q4_0, Q5_0, Q8_0 = 2, 6, 8
@@ -83,11 +83,6 @@ def quant_shape(weight_type: int, n: int, row_bytes: int) -> tuple[int, int]:
     if row_bytes % bb:
         raise ValueError(f"{row_bytes} bytes per row is not a whole number of {bb}-byte blocks of type {weight_type}")
     return n, row_bytes // bb * bw
-
-
-def _stream(device: torch.device) -> int:
-    """The device's current stream as a raw handle (no Stream object is made)."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_gpu(t: torch.Tensor, what: str) -> None:
@@ -349,27 +344,6 @@ def fused_mul_mat_gguf_grouped_out(x: torch.Tensor, packed: torch.Tensor, descs:
     """As fused_mul_mat_gguf_grouped, writing into `out` (bf16 [M, n_total], unit column stride:
     e.g. the column slice of a wider layer output that this run's shards own)."""
     _grouped_into(x, packed, descs, plans, workspace, bias, out)
-
-
-def _direct(*tensors: torch.Tensor | None) -> bool:
-    """Whether an eager call may go to the library without the dispatcher: nothing traces, transforms
-    or intercepts it (compile, fx and jit tracing, dispatch and function modes, functorch, forward-mode
-    AD), no profiler records the ops, and no tensor needs more than its data pointer (subclasses, lazy
-    negation, functional and zero tensors, autograd).  The dispatcher's share of a custom op call with
-    its two list arguments is about 30 us, several times the launch of a small layer (8 us of GPU time
-    for a 4096 x 4096 Q8_0 layer at one row, whose eager call took 46 us).  An ExecutionTraceObserver
-    that runs without a profiler cannot be seen from here: it misses the op."""
-    if (torch.compiler.is_compiling() or profiler._is_profiler_enabled or torch.autograd._profiler_enabled()
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
-            or forward_ad._current_level >= 0):
-        return False
-    grad = torch.is_grad_enabled()
-    for t in tensors:
-        if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or t.is_neg()
-                              or t._is_zerotensor() or torch._is_functional_tensor(t) or (grad and t.requires_grad)):
-            return False
-    return True
 
 
 def mul_mat_grouped(x: torch.Tensor, gl: GroupedLayer, bias: torch.Tensor | None = None,

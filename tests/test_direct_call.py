@@ -79,6 +79,35 @@ def test_a_profiler_sees_the_op():
     assert seen == [False] * 3 and _direct(x)
 
 
+@pytest.mark.parametrize("where,name", [
+    (torch._C, "_len_torch_dispatch_stack"), (torch._C, "_len_torch_function_stack"), (torch._C, "_get_tracing_state"),
+    (torch._C._functorch, "peek_interpreter_stack"), (torch.autograd, "_profiler_enabled"),
+    (torch, "_is_functional_tensor"), (fwad, "_current_level"), (torch.autograd.profiler, "_is_profiler_enabled"),
+], ids=lambda v: v if isinstance(v, str) else "")
+def test_a_torch_without_one_of_the_names_takes_the_op(monkeypatch, where, name):
+    import importlib.util
+
+    from gguf_hip import eager
+
+    monkeypatch.delattr(where, name)
+    spec = importlib.util.spec_from_file_location("eager_without", eager.__file__)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    no = mod.direct(torch.zeros(1))
+    monkeypatch.undo()
+    assert no is False and eager.direct(torch.zeros(1))
+
+
+def test_the_stream_without_the_raw_handle(monkeypatch):
+    import types
+
+    from gguf_hip import eager
+
+    monkeypatch.setattr(eager, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=77))
+    assert eager.stream(torch.device("cuda", 0)) == 77
+
+
 @pytest.mark.gpu
 def test_direct_and_dispatched_calls_agree(dev):
     import gguf_hip
