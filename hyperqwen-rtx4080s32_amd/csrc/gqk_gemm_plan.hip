@@ -31,7 +31,8 @@ static int64_t slot_bytes(int mb, int nr, int wk) { return (int64_t)((4 * mb + w
 // x, k-group combine, store) and its k-steps; split tiles add the exchange of partials.  The step times
 // (us, one workgroup per CU) are fits to Q4_K and Q6_K launches over nine shapes (1000 x 4096 to
 // 34816 x 5120, 5120 x 17408) at 40-1024 rows, each geometry forced in turn: the pick is within 5% of
-// the best geometry in nine cases of ten and 1.2 times it at worst.  Why more than one geometry (us,
+// the best geometry in nine cases of ten and 1.2 times it at worst (so for eleven types and mixed layers,
+// profiles/gemm_geometry_sweep.md).  Why more than one geometry (us,
 // Q4_K): at 64 rows 34816 x 5120 takes 41.5 with 5 row blocks (218 workgroups, one round), 60.7 with 4
 // (272: two rounds) and 52.0 with 8; 5120 x 17408 28.4 with 2 row blocks split 3 ways, 31.2 with 4
 // split 6 ways, whose last contributor sums twice the partials; at 128 rows 38.6 (4 row blocks, 128
@@ -53,7 +54,13 @@ static GemmPick pick(int bm, int n_desc, int M, int nb, int cus) {
       p.gsk = (int)stream_k_workgroups(cus, R, nb);
       p.grid = (int)(W >= cus ? cus : p.gsk);
       p.slots = R ? R + p.gsk - 1 : 0;
-      us = 10. + (double)W * 4 * nb * step_us / p.grid + (R ? exch_us : 0.);
+      // The whole rounds, then the remainder tiles on gsk workgroups: few of them where R or nb is small,
+      // so that such a tail lasts as long as a round.  Spread over every workgroup in the estimate (as it
+      // was) it hid: us, the form taken then -> now, at R = 2-56: Q4_K 33024 x 5120 at 384 rows 186 -> 176,
+      // Q5_K 24778 x 1280 at 563 90 -> 70, IQ4_XS 18043 x 512 at 1094 76 -> 53, Q8_0 24140 x 256 at 564 77
+      // -> 32.  After whole rounds the exchange waits for less (12 of 16 us: 16 took others 5-8% slower).
+      us = 10. + (double)(W / cus) * 4 * nb * step_us +
+           (R ? (double)R * nb / p.gsk * 4 * step_us + (W >= cus ? 0.75 : 1.) * exch_us : 0.);
     } else {
       int64_t S = 1;
       if (W < cus) S = std::max<int64_t>(1, std::min<int64_t>({cus / W, nb / wk, 8}));
@@ -93,6 +100,16 @@ int64_t gemm_workspace_max() {
   const int cus = gb_cus();
   if (cus <= 0) return -1;
   return GQK_CTR_BYTES + (int64_t)(2 * cus - 2) * slot_bytes(8, 8, 1);
+}
+
+int gemm_pick(int bm, int n_desc, int M, int nb, int cus, int32_t* out) {
+  if (bm != 64 && bm != 128 && bm != 256) return GQK_ERR_FORM;
+  if (cus == 0) cus = gb_cus();
+  if (cus <= 0) return GQK_ERR_HIP;
+  const GemmPick p = pick(bm, n_desc, M, nb, cus);
+  const int32_t v[7] = {p.mb, p.nr, p.wk, p.S, p.mb == 8 ? p.gsk : 0, p.grid, (int32_t)p.slots};
+  for (int i = 0; i < 7; ++i) out[i] = v[i];
+  return GQK_OK;
 }
 
 int launch_gemm(const uint8_t* packed, const int32_t* desc, int n_desc, int types_mask, const void* x, int64_t ldx,

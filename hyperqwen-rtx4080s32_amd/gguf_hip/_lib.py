@@ -25,7 +25,7 @@ GQK_DTYPE_F32, GQK_DTYPE_BF16, GQK_DTYPE_F16 = 0, 1, 2
 # every entry point include/gguf_hip.h declares
 EXPORTS = ("gqk_last_error", "gqk_version", "gqk_type_info", "gqk_dequantize", "gqk_dequantize_tiles",
            "gqk_tiles_bytes", "gqk_repack", "gqk_unrepack", "gqk_plan", "gqk_linear_workspace_bytes",
-           "gqk_workspace_bytes_max", "gqk_linear", "gqk_linear_noalloc", "gqk_ggml_type_size",
+           "gqk_gemm_pick", "gqk_workspace_bytes_max", "gqk_linear", "gqk_linear_noalloc", "gqk_ggml_type_size",
            "gqk_gguf_open", "gqk_gguf_close", "gqk_gguf_info", "gqk_gguf_tensor_at", "gqk_gguf_find_tensor",
            "gqk_gguf_kv_at", "gqk_gguf_find_kv", "gqk_gguf_kv_string", "gqk_gguf_upload_tiles", "gqk_read_floor")
 
@@ -88,6 +88,7 @@ def _load() -> ctypes.CDLL:
         "gqk_plan": (i32, [ctypes.POINTER(GqkShard), i32, i64, i32, i32, i32, ctypes.POINTER(ctypes.c_int32), i64,
                            ctypes.POINTER(GqkPlanInfo)]),
         "gqk_linear_workspace_bytes": (i64, [ctypes.POINTER(GqkPlanInfo), i32]),
+        "gqk_gemm_pick": (i32, [ctypes.POINTER(GqkPlanInfo), i32, i32, ctypes.POINTER(ctypes.c_int32)]),
         "gqk_workspace_bytes_max": (i64, []),
         "gqk_linear": (i32, [vp, vp, ctypes.POINTER(GqkPlanInfo), vp, i64, i32, vp, i64, vp, vp, i64, vp]),
         "gqk_linear_noalloc": (i32, [vp, vp, ctypes.POINTER(GqkPlanInfo), vp, i64, i32, vp, i64, vp, vp]),

@@ -200,6 +200,13 @@ def plan(shards: list[tuple[int, int, int]], K: int, M: int, target_wgs: int = 0
     return info, desc
 
 
+def gemm_pick(info: GqkPlanInfo, M: int, cus: int = 0) -> dict[str, int]:
+    """The tile geometry and schedule a GEMM plan's launch takes at M rows (gqk_gemm_pick)."""
+    out = (ctypes.c_int32 * 7)()
+    check(lib.gqk_gemm_pick(ctypes.byref(info), M, cus, out), "gemm_pick")
+    return dict(zip(("mb", "nr", "wk", "split", "tail_wgs", "wgs", "slots"), out))
+
+
 @dataclass
 class GroupedLayer:
     """A run of shards packed into one buffer with the plans of every batch-row bucket (the

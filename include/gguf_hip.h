@@ -126,6 +126,13 @@ int gqk_plan(const gqk_shard* shards, int nshards, int64_t K, int M, int target_
  * partial tiles, which depends on M and on the current device's CU count.  Replaces the reference's transient split-K partials (gguf-plugin/gluon/tiles_grouped.py:1233-1238). */
 int64_t gqk_linear_workspace_bytes(const gqk_plan_info* info, int M);
 
+/* The tile geometry and schedule gqk_linear takes for a GEMM plan at M batch rows on a device of `cus`
+ * compute units (0: the current device), on the host: out[7] = 32-token blocks per tile, 32-row blocks
+ * per tile, k-groups of waves, k-splits per tile (workgroups; 1 for the persistent form of 8 x 8 blocks),
+ * workgroups of the persistent form's remainder tiles, workgroups launched, fp32 partial slots.  For
+ * tests and measurements; no counterpart in the reference. */
+int gqk_gemm_pick(const gqk_plan_info* info, int M, int cus, int32_t* out);
+
 /* Workspace bytes that serve every GEMM plan at any M on the current device (< 0: error): one
  * buffer of this size (or of a layer's GEMV workspace_bytes, if larger) serves every layer on the
  * device, as calls on one stream never overlap.  No counterpart in the reference, whose split-K
