@@ -79,7 +79,7 @@ def test_config4_prefill_gemm(dev, wt):
 def test_reference_wide_form_edges(dev, wt):
     """The reference's wide-form edge list (gguf-plugin/test_gluon_wide_gpu.py:37-39): ffn_gate,
     attn_k / attn_v, a k / v row count with ffn_down's K, and a 48-row shard (a partial tile), at
-    the row counts around every GEMM tile form's boundary."""
+    the row counts around the GEMM plans' boundaries."""
     for i, (n, K) in enumerate([(17408, 5120), (1024, 5120), (1024, 17408), (48, 5120)]):
         _check_shard(dev, wt, n, K, Ms=(33, 64, 65, 128, 129, 2048), seed=400 + 10 * wt + i)
 
@@ -89,8 +89,8 @@ def test_config5_mixed_type_layers(dev, layer):
     """BASELINE config 5 at its layer shapes: decoder layers of the seeded 64-layer type draw
     (the one bench_configs.py times), each as one mixed-type grouped launch over qkv 7168 / o_proj
     5120 / gate_up 34816 rows at K = 5120 plus down 5120 x 17408, at M = 1, 8, 12, 32, 64, 100 (the
-    mixed-type GEMV, with the 16 x 16 x 32 form's types at 12, and every small GEMM form, x staged
-    by direct-to-LDS loads at 100): every
+    mixed-type GEMV, with the 16 x 16 x 32 form's types at 12, the mid form, and the GEMM with 64-
+    and 128-token tiles): every
     shard's rows pinned bit-exact against the oracle on a subset, and the launches against an fp32
     matmul of the dequantized weights within 1e-2."""
     import gguf_hip

@@ -1,6 +1,7 @@
 """The GEMM's tile geometries at the sizes where they can go wrong: token and row remainders, row blocks
 past the last descriptor row, k-groups with unequal (or no) super-blocks, split and unsplit tiles,
-mixed types inside a workgroup, x rows further apart than 32-bit offsets reach.  Against the fp64
+mixed types inside a workgroup, x rows further apart than 32-bit offsets reach.  Which geometry a case
+runs is asserted (ops.gemm_pick; the sizes are for 256 compute units).  Against the fp64
 product of the oracle's weights: bf16 keeps eight bits, so rounding to nearest moves a value by at most
 2^-8 of it; one rounding of each weight and of y moves an output by at most 2^-8 (sum |x w| + |y|), fp32
 accumulation by far less (the 1 %); over all outputs the error is under 1e-2."""
@@ -32,10 +33,44 @@ def _layer(dev, shards, K, seed, cus=0):
                                [wt for wt, _ in shards], cus=cus), wf
 
 
+def _pick(gl, M):
+    from gguf_hip import ops
+
+    i = ops._pick_plan(gl.plans, M)
+    info = ops.GqkPlanInfo.from_tuple(gl.plans[i * ops._NPLAN:][:ops._NPLAN])
+    return info, ops.gemm_pick(info, M)
+
+
+def _check(gl, x, wf, bias):
+    """y of the layer (wf: its fp64 weights on the GPU) against its bound, three bit-identical repeats, and
+    the counters back at zero."""
+    import gguf_hip
+
+    y = gguf_hip.mul_mat_grouped(x, gl, bias)
+    ref = x.double() @ wf.T + bias.double()
+    bound = 2.0 ** -8 * (x.double().abs() @ wf.abs().T + ref.abs())
+    worst = float(((y.double() - ref).abs() / (bound + 1e-30)).max())
+    print("error over its bound", worst, flush=True)
+    assert worst <= 1.01 and float((y.double() - ref).norm()) <= 1e-2 * float(ref.norm())
+    for _ in range(3):
+        assert torch.equal(gguf_hip.mul_mat_grouped(x, gl, bias), y)
+    torch.cuda.synchronize()
+    assert int(gl.workspace[:65536].abs().sum()) == 0
+
+
+def _random_layer(dev, ns, types, K):
+    import gguf_hip
+    from gguf_hip.synth import random_shard
+
+    raws = [random_shard(n, K, t, dev, seed=t) for n, t in zip(ns, types)]
+    wf = torch.cat([gguf_hip.dequantize(w, t, (n, K)) for w, n, t in zip(raws, ns, types)]).double()
+    return gguf_hip.pack_layer(raws, ns, list(types)), wf
+
+
 @pytest.mark.parametrize("shards,nbk", [
     ([(G.Q4_K, 1)], 1),                                     # one row, fewer super-blocks than k-groups
     ([(G.Q3_K, 97)], 2),
-    ([(G.Q6_K, 161), (G.IQ3_S, 31)], 3),                    # a workgroup's waves on different types
+    ([(G.Q6_K, 161), (G.IQ3_S, 31)], 3),                    # descriptor rows of different types
     ([(G.Q8_0, 330)], 5),
     ([(G.IQ4_XS, 640), (G.Q2_K, 70), (G.Q5_0, 129)], 7),
     ([(G.Q5_K, 2100)], 9),
@@ -43,6 +78,7 @@ def _layer(dev, shards, K, seed, cus=0):
     ([(G.Q4_K, 1097)], 4),                                  # unsplit: eights of tiles and a rest, dealt to XCDs
 ])
 def test_geometries(dev, shards, nbk):
+    """Layers up to 2,100 rows: the 64 x 64 geometry, unsplit and split, against the oracle."""
     import gguf_hip
 
     K = 256 * nbk
@@ -59,42 +95,48 @@ def test_geometries(dev, shards, nbk):
     assert int(gl.workspace[:65536].abs().sum()) == 0
 
 
-@pytest.mark.parametrize("n0,nbk,M", [
-    (600, 20, 760),    # remainder tiles only, each shared by several workgroups
-    (800, 1, 1801),    # whole tiles dealt to the workgroups, then remainder tiles of one super-block
+@pytest.mark.parametrize("geo,split,n0,nbk,M", [
+    ((2, 2, 4), False, 3, 1, 33), ((2, 2, 4), False, 3, 5, 33), ((2, 2, 4), True, 3, 9, 33),
+    ((2, 4, 4), False, 3, 3, 761), ((2, 4, 4), False, 3, 7, 761), ((2, 4, 4), True, 3, 20, 221),
+    # five waves of row blocks: a workgroup straddles descriptor rows, so its waves decode different types
+    ((2, 5, 3), False, 3, 3, 851), ((2, 5, 3), False, 2900, 1, 33), ((2, 5, 3), False, 2900, 5, 33),
+    ((4, 4, 2), False, 3, 1, 761), ((4, 4, 2), False, 3, 3, 941), ((4, 4, 2), True, 3, 20, 761),
+    ((4, 5, 2), False, 3, 1, 1481), ((4, 5, 2), False, 3, 3, 1481), ((4, 5, 2), True, 3, 20, 851),
+    ((8, 8, 1), False, 600, 20, 760),   # remainder tiles only, each shared by several workgroups
+    ((8, 8, 1), False, 800, 1, 1801),   # whole tiles dealt to the workgroups, then remainder tiles of one super-block
+    ((8, 8, 1), False, 3, 12, 1841),
 ])
-def test_persistent_tiles_of_every_type(dev, n0, nbk, M):
-    """The 256 x 256 form on a layer with a shard of each type: consecutive tiles of a workgroup have
-    different types, and the remainder tiles' partials are of all types."""
-    import ctypes
-
-    import gguf_hip
-    from gguf_hip import _lib, ops
-    from gguf_hip.synth import random_shard
-
-    K, ns = 256 * nbk, [n0 + 7 * i for i in range(len(G.ALL_TYPES))]
-    raws = [random_shard(n, K, t, dev, seed=t) for n, t in zip(ns, G.ALL_TYPES)]
-    wf = torch.cat([gguf_hip.dequantize(w, t, (n, K)) for w, n, t in zip(raws, ns, G.ALL_TYPES)]).double()
-    gl = gguf_hip.pack_layer(raws, ns, list(G.ALL_TYPES))
-    i = ops._pick_plan(gl.plans, M)
-    info = ops.GqkPlanInfo.from_tuple(gl.plans[i * ops._NPLAN:][:ops._NPLAN])
-    slots = (_lib.lib.gqk_linear_workspace_bytes(ctypes.byref(info), M) - info.ctr_bytes) / (256 * 256 * 4)
-    assert info.bm == 256 and slots > 0 and slots % 1 == 0     # only this form's slots hold 256 x 256 sums
+def test_mixed_layers_on_every_geometry(dev, geo, split, n0, nbk, M):
+    """A layer with a ragged shard of each type (the mixed-type build), fewer super-blocks than k-groups,
+    k-groups of unequal length, split tiles."""
+    ns, K = [n0 + 7 * i for i in range(len(G.ALL_TYPES))], 256 * nbk
+    gl, wf = _random_layer(dev, ns, G.ALL_TYPES, K)
+    info, p = _pick(gl, M)
+    assert info.types_mask == 0 and (p["mb"], p["nr"], p["wk"]) == geo and (p["split"] > 1) == split, p
+    assert geo[0] < 8 or p["slots"] > 0, p
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(dev)
-    bias = torch.randn(gl.n_total, device=dev).to(torch.bfloat16)
-    print(n0, nbk, M, slots, flush=True)
-    y = gguf_hip.mul_mat_grouped(x, gl, bias)
-    ref = x.double() @ wf.T + bias.double()
-    mag = x.double().abs() @ wf.abs().T
-    err = (y.double() - ref).abs()
-    worst = float((err / (2.0 ** -8 * (mag + ref.abs()) + 1e-30)).max())
-    print("error over its bound", worst, flush=True)
-    assert worst <= 1.01
-    assert float(err.norm()) <= 1e-2 * float(ref.norm())
-    for _ in range(3):
-        assert torch.equal(gguf_hip.mul_mat_grouped(x, gl, bias), y)
-    torch.cuda.synchronize()
-    assert int(gl.workspace[:info.ctr_bytes // 4].abs().sum()) == 0
+    print(geo, p, flush=True)
+    _check(gl, x, wf, torch.randn(gl.n_total, device=dev).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("geo,split,n,nbk,M", [
+    ((2, 2, 4), False, 97, 5, 34), ((2, 2, 4), True, 97, 9, 34), ((2, 4, 4), False, 257, 5, 2111),
+    ((2, 4, 4), True, 33, 20, 1391), ((2, 5, 3), False, 33000, 4, 33), ((4, 4, 2), False, 20600, 3, 72),
+    ((4, 4, 2), True, 257, 20, 2111), ((4, 5, 2), False, 16500, 3, 131), ((4, 5, 2), True, 16500, 20, 72),
+    ((8, 8, 1), False, 24700, 3, 401),
+])
+def test_each_type_on_every_geometry(dev, geo, split, n, nbk, M):
+    """The single-type builds: the barrier's count of loads in flight depends on the geometry and on the
+    type's loads."""
+    K = 256 * nbk
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(dev)
+    for t in G.ALL_TYPES:
+        gl, wf = _random_layer(dev, [n], [t], K)
+        info, p = _pick(gl, M)
+        assert info.types_mask == t and (p["mb"], p["nr"], p["wk"]) == geo and (p["split"] > 1) == split, p
+        assert geo[0] < 8 or p["slots"] > p["tail_wgs"], p
+        print(G.NAMES[t], p, flush=True)
+        _check(gl, x, wf, torch.randn(n, device=dev).to(torch.bfloat16))
 
 
 def _launches(fn):
@@ -118,10 +160,8 @@ def test_rows_far_apart(dev, ldx):
     slab, _ = _layer(dev, [(G.Q4_K, 130), (G.IQ3_S, 64)], K, 3, cus=8)
     wide = None
     if ldx < 1 << 23:
-        from gguf_hip.synth import random_shard
-
-        ns = [800 + 7 * i for i in range(len(G.ALL_TYPES))]
-        wide = gguf_hip.pack_layer([random_shard(n, K, t, dev, seed=t) for n, t in zip(ns, G.ALL_TYPES)], ns, list(G.ALL_TYPES))
+        wide, _ = _random_layer(dev, [800 + 7 * i for i in range(len(G.ALL_TYPES))], G.ALL_TYPES, K)
+        assert _pick(wide, 1801)[1]["mb"] == 8
     for gl, M in ((small, 3), (small, 18), (slab, 32), (small, 34), (small, 41), (wide, 1801)):
         if gl is None:
             continue

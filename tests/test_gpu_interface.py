@@ -197,13 +197,13 @@ def test_dequantize_tiles_one_pass(dev, wt):
 
 def test_shared_workspace_many_layers(dev):
     """One workspace per device serves every layer: 100 mixed-type layers share it, each checked
-    at a GEMV M (split-K), a 17-row and a stream-K GEMM M, twice for bit identity, with the
+    at a GEMV M (split-K), a 17-row and a split GEMM M, twice for bit identity, with the
     counters back at zero at the end."""
     import gguf_hip
     from gguf_hip import ops
 
     rng = np.random.default_rng(33)
-    K = 1024
+    K = 2304
     types = [G.Q4_K, G.Q6_K, G.IQ4_XS, G.Q8_0, G.Q3_K, G.IQ3_S, G.Q5_0]
     layers = []
     for i in range(100):
@@ -214,6 +214,9 @@ def test_shared_workspace_many_layers(dev):
         layers.append((gl, np.concatenate([G.dequantize(r, wt) for r, (wt, _) in zip(raws, sh)])))
     ws = layers[0][0].workspace
     assert all(gl.workspace is ws for gl, _ in layers)
+    i = ops._pick_plan(layers[0][0].plans, 300)
+    for gl, _ in layers:
+        assert ops.gemm_pick(ops.GqkPlanInfo.from_tuple(gl.plans[i * ops._NPLAN:][:ops._NPLAN]), 300)["slots"] > 0
     print(f"shared workspace: {ws.numel() * 4 / 2**20:.1f} MiB for {len(layers)} layers")
     before = torch.cuda.memory_allocated(dev)
     for M in (6, 17, 300):
@@ -231,10 +234,12 @@ def test_shared_workspace_many_layers(dev):
 
 
 def test_graph_then_larger_eager_call_then_replay(dev):
-    """A graph captured at a GEMV M, then eager calls at a large GEMM M on the same and another
-    layer (the stream-K partials fill the shared workspace), then the graph replayed: the
-    workspace never moved, so the replay still matches its eager result."""
+    """A graph captured at a GEMV M, then eager calls at large GEMM Ms on the same and other layers (one
+    of them with 338 stream-K partial slots, 88 MB of the shared workspace), then the graph
+    replayed: the workspace never moved, so the replay still matches its eager result."""
     import gguf_hip
+    from gguf_hip import ops
+    from gguf_hip.synth import random_shard
 
     rng = np.random.default_rng(34)
     K = 2560
@@ -242,6 +247,11 @@ def test_graph_then_larger_eager_call_then_replay(dev):
     raw_b = G.random_blocks(rng, 900, K, G.Q6_K)
     gla = gguf_hip.pack_layer([torch.from_numpy(raw_a).to(dev)], [700], [G.Q4_K], target_wgs=4096)
     glb = gguf_hip.pack_layer([torch.from_numpy(raw_b).to(dev)], [900], [G.Q6_K])
+    Wc = random_shard(24700, 768, G.Q5_K, dev)
+    glc = gguf_hip.pack_layer([Wc], [24700], [G.Q5_K])
+    i = ops._pick_plan(glc.plans, 401)
+    pick = ops.gemm_pick(ops.GqkPlanInfo.from_tuple(glc.plans[i * ops._NPLAN:][:ops._NPLAN]), 401)
+    assert pick["mb"] == 8 and pick["slots"] == 338
     ws_ptr = gla.workspace.data_ptr()
     x8 = _x(8, K, 8, dev)
     eager = gguf_hip.mul_mat_grouped(x8, gla)
@@ -255,6 +265,10 @@ def test_graph_then_larger_eager_call_then_replay(dev):
             yb = gguf_hip.mul_mat_grouped(xb, gl)
             if M == 1000:
                 assert G.rel_err(yb[:64].float().cpu().numpy(), _ref(xb[:64], G.dequantize(raw, wt))) < TOL
+        xc = _x(401, 768, M, dev)
+        yc = gguf_hip.mul_mat_grouped(xc, glc)
+        ref = xc.float() @ gguf_hip.dequantize(Wc, G.Q5_K, (24700, 768)).T
+        assert float(((yc.float() - ref).abs() / ref.abs().amax(dim=1, keepdim=True)).amax()) < TOL
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, eager), M

@@ -116,8 +116,8 @@ def test_gemv_tail_tiles_split(dev, wt):
 def test_graph_replay_matches_eager(dev):
     """The grouped op captured in one HIP graph, as a serving loop (and bench.py) runs it: the
     GEMV with split-K partials and in-kernel counters, the GEMV with a split tail, with a fused
-    bias, the mid form (17..32 rows) with split K, and the stream-K GEMM in its 64-row and 256-row
-    forms.  Five replays, each after new x
+    bias, the mid form (17..32 rows) with split K, the GEMM with split tiles and its 256 x 256
+    form with shared remainder tiles.  Five replays, each after new x
     is copied into the captured inputs, followed by eager launches of the same layers (sharing
     the layers' workspaces) and a host synchronisation: every replay is bit-identical to the
     eager result on the same x, which matches the oracle, and the counters end at zero (they are
@@ -130,8 +130,9 @@ def test_graph_replay_matches_eager(dev):
         (G.Q6_K, 900, 12 * 256, 1, 0, True),         # GEMV, split K, fused bf16 bias
         (G.IQ4_XS, 64 * 9 + 17, 16 * 256, 5, 16, False),   # GEMV, whole tiles + split tail
         (G.Q5_K, 1000, 2048, 20, 0, False),          # mid form, split K
-        (G.Q6_K, 1000, 2048, 40, 0, False),          # GEMM 64 x 128, stream-K only
-        (G.Q4_K, 1000, 2048, 300, 0, True),          # GEMM 256 x 256, stream-K, bias
+        (G.Q6_K, 1000, 2048, 40, 0, False),          # GEMM 64 x 64, tiles split in two
+        (G.Q4_K, 1000, 2048, 300, 0, True),          # the same at five token blocks, bias
+        (G.Q5_K, 24700, 768, 401, 0, True),          # GEMM 256 x 256, stream-K, bias
     ]
     layers, xs, biases, wfs = [], [], [], []
     for i, (wt, n, K, M, tw, has_bias) in enumerate(cases):
@@ -144,6 +145,9 @@ def test_graph_replay_matches_eager(dev):
         info = gguf_hip.ops.GqkPlanInfo.from_tuple(
             gl.plans[gguf_hip.ops._pick_plan(gl.plans, M) * gguf_hip.ops._NPLAN:][:gguf_hip.ops._NPLAN])
         assert info.form == (1 if M <= 32 else 2) and (M > 32 or info.split > 1), (G.NAMES[wt], M)
+        if M > 32:                                   # every GEMM case exchanges partials
+            p = gguf_hip.ops.gemm_pick(info, M)
+            assert p["slots"] > p["tail_wgs"] and (p["mb"] == 8) == (n == 24700), p
 
     def run():
         return [gguf_hip.mul_mat_grouped(x, gl, b) for x, gl, b in zip(xs, layers, biases)]
@@ -202,7 +206,7 @@ def test_random_layers_match_reference(dev):
 
 
 def test_one_workspace_serves_every_form(dev):
-    """One layer workspace across the GEMV and mid form (split tiles) and the GEMM forms (stream-K
+    """One layer workspace across the GEMV and mid form (split tiles) and the GEMM (split tiles'
     partials) in an order where each form's partials would land on another form's counters if
     the counter regions differed: every call matches the oracle and repeats bit-identically,
     and the counters end at zero."""
@@ -230,7 +234,7 @@ def test_one_workspace_serves_every_form(dev):
 def test_mixed_layer_one_launch(dev):
     """A merged layer of five types in one grouped launch.  GEMV (split 1): every shard's columns
     are bit-identical to its own launch (the reference's mixed-layer identity at a fixed split,
-    gguf-plugin/test_gluon_kq_gpu.py:172-195).  GEMM: the stream-K k-ranges of a tile depend on
+    gguf-plugin/test_gluon_kq_gpu.py:172-195).  GEMM: the k-splits of a tile depend on
     the launch's whole tile count, so a shard's fp32 partial sums may associate differently
     alone: its columns match the oracle and stay within bf16 rounding of its own launch."""
     import gguf_hip
@@ -467,8 +471,8 @@ def test_gemv_slab_form_mixed_layer(dev):
 
 
 def test_fused_bias(dev):
-    """A bf16 bias is added in the kernels' epilogue (direct GEMV store, split-K fixup, GEMM and
-    stream-K fixup): a zero bias changes no bit, a random one matches oracle + bias; an fp32 bias
+    """A bf16 bias is added in the kernels' epilogue (direct GEMV store, split-K fixup, split
+    GEMM): a zero bias changes no bit, a random one matches oracle + bias; an fp32 bias
     is added afterwards."""
     import gguf_hip
 
@@ -526,28 +530,31 @@ def test_baseline_config1_q8_0(dev):
     assert e < TOL, e
 
 
-@pytest.mark.parametrize("n,K,M", [(1000, 2048, 300), (1000, 2048, 2148), (16384, 512, 1100),
-                                   (1000, 2048, 40), (16384, 512, 100), (70000, 256, 64), (70000, 256, 120),
-                                   (1000, 2048, 33), (5120, 5120, 48), (200000, 256, 40)],
-                         ids=str)
+@pytest.mark.parametrize("n,K,M,geo,shared", [
+    (1000, 2048, 300, (2, 2, 4), True), (1000, 2048, 2148, (4, 4, 2), False), (16384, 512, 1100, (4, 5, 2), False),
+    (1000, 2048, 40, (2, 2, 4), True), (16384, 512, 100, (4, 4, 2), False), (70000, 256, 64, (2, 5, 3), False),
+    (70000, 256, 120, (4, 5, 2), False), (1000, 2048, 33, (2, 2, 4), True), (5120, 5120, 48, (2, 2, 4), True),
+    (200000, 256, 40, (2, 5, 3), False),
+    (17391, 5120, 2040, (8, 8, 1), True), (5101, 17408, 500, (8, 8, 1), True), (33000, 256, 401, (8, 8, 1), False),
+], ids=str)
 @pytest.mark.parametrize("wt", [G.Q5_K, G.Q4_K, G.Q8_0], ids=lambda t: G.NAMES[t])
-def test_gemm_stream_k_schedule(dev, n, K, M, wt):
-    """The GEMM forms' persistent schedule (256 x 256 tiles above 128 rows, except 129..384 rows of a
-    layer with few 256-row groups, which keep 128 x 128 (1000 rows at M = 300 here); 128 x 128 and
-    64 x 128 at 65..128 and 33..64): whole tiles dealt to the workgroups, the remainder
-    tiles' k-steps split over up to all of them (stream-K, >= 16 steps each, <= 6 per tile) and
-    combined in k order by the last contributor.  Small grids are all remainder; the 16384-row
-    case at M=1100 and the 70000- and 200000-row cases mix both phases.  The 256 x 256 tile runs
-    with its waves 2 x 4 for Q5_K, 4 x 2 with x staged by direct-to-LDS loads for Q4_K and 4 x 2
-    with x through registers for Q8_0; the 128 x 128 form stages x by direct loads.  Checked
-    against an fp32 matmul of the GPU-dequantized weights (pinned bit-exact by the dequant
-    tests), repeated launches bit-identical, counters back at zero."""
+def test_gemm_schedule(dev, n, K, M, geo, shared, wt):
+    """The GEMM's schedules: one workgroup per tile and k-split (geometries below 256 tokens), split where
+    the tiles are fewer than the CUs and K is long; the 256 x 256 form persistent, whole tiles dealt to the
+    workgroups and the remainder tiles' super-blocks split over some of them (stream-K), remainder
+    tiles only or both phases.  Partials of a shared tile are combined in k order by the last
+    contributor.  Checked against an fp32 matmul of the GPU-dequantized weights (pinned bit-exact by
+    the dequant tests), repeated launches bit-identical, counters back at zero; geometry and sharing
+    are asserted (for 256 CUs)."""
     import gguf_hip
     from gguf_hip.synth import random_shard
 
     W = random_shard(n, K, wt, dev, seed=n + M)
     wf = gguf_hip.dequantize(W, wt, (n, K), torch.float32)
     gl = gguf_hip.pack_layer([W], [n], [wt])
+    i = gguf_hip.ops._pick_plan(gl.plans, M)
+    p = gguf_hip.ops.gemm_pick(gguf_hip.ops.GqkPlanInfo.from_tuple(gl.plans[i * gguf_hip.ops._NPLAN:][:gguf_hip.ops._NPLAN]), M)
+    assert (p["mb"], p["nr"], p["wk"]) == geo and (p["split"] > 1 or (p["mb"] == 8 and p["tail_wgs"] > 1)) == shared, p
     x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(torch.bfloat16)
     y = gguf_hip.mul_mat_grouped(x, gl)
     ref = x.float() @ wf.T
@@ -564,27 +571,33 @@ def test_gemm_stream_k_schedule(dev, n, K, M, wt):
 def test_strided_activations_every_form(dev, wt):
     """x as a column slice of a wider buffer (row stride K + 24, 16-byte aligned start) goes to the
     kernels as is, in every form: GEMV (M <= 16; at 9-16 rows Q8_0 / IQ4_XS read it straight from
-    global memory in the 16 x 16 x 32 form), the mid form (17..32 rows, x read straight from global
-    memory) and the three GEMM tiles, with x staged through
-    registers (Q6_K, Q8_0 in the 256 x 256 form) or by direct-to-LDS loads (the 128 x 128 form,
-    Q4_K in the 256 x 256 form), full and partial token blocks.  Each result is bit-identical to
-    the one from a contiguous copy of x."""
+    global memory in the 16 x 16 x 32 form), the mid form (17..32 rows) and the GEMM's six
+    geometries (x by direct-to-LDS loads), full and partial token blocks.  Each result is
+    bit-identical to the one from a contiguous copy of x."""
     import gguf_hip
     from gguf_hip.synth import random_shard
 
-    n, K = 300, 2048
-    W = random_shard(n, K, wt, dev, seed=77 + wt)
-    gl = gguf_hip.pack_layer([W], [n], [wt])
-    wf = gguf_hip.dequantize(W, wt, (n, K), torch.float32)
-    for M in (8, 12, 20, 48, 100, 256, 300):
-        big = torch.randn(M, K + 24, device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(torch.bfloat16)
-        xs = big[:, 8:8 + K]
-        assert xs.stride(0) == K + 24 and xs.data_ptr() % 16 == 0
-        y = gguf_hip.mul_mat_grouped(xs, gl)
-        assert torch.equal(y, gguf_hip.mul_mat_grouped(xs.contiguous(), gl)), (G.NAMES[wt], M)
-        ref = xs.float() @ wf.T
-        e = float(((y.float() - ref).abs() / ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)).amax())
-        assert e < TOL, (G.NAMES[wt], M, e)
+    seen = set()
+    for n, K, Ms in ((300, 2048, (8, 12, 20, 48, 100, 256, 300)), (33000, 256, (40,)), (16500, 256, (131,)),
+                     (257, 768, (2111,)), (257, 512, (2111,)), (24700, 768, (401,))):
+        W = random_shard(n, K, wt, dev, seed=77 + wt)
+        gl = gguf_hip.pack_layer([W], [n], [wt])
+        wf = gguf_hip.dequantize(W, wt, (n, K), torch.float32)
+        for M in Ms:
+            i = gguf_hip.ops._pick_plan(gl.plans, M)
+            info = gguf_hip.ops.GqkPlanInfo.from_tuple(gl.plans[i * gguf_hip.ops._NPLAN:][:gguf_hip.ops._NPLAN])
+            if M > 32:
+                p = gguf_hip.ops.gemm_pick(info, M)
+                seen.add((p["mb"], p["nr"]))
+            big = torch.randn(M, K + 24, device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(torch.bfloat16)
+            xs = big[:, 8:8 + K]
+            assert xs.stride(0) == K + 24 and xs.data_ptr() % 16 == 0
+            y = gguf_hip.mul_mat_grouped(xs, gl)
+            assert torch.equal(y, gguf_hip.mul_mat_grouped(xs.contiguous(), gl)), (G.NAMES[wt], M)
+            ref = xs.float() @ wf.T
+            e = float(((y.float() - ref).abs() / ref.abs().amax(dim=1, keepdim=True).clamp(min=1e-30)).amax())
+            assert e < TOL, (G.NAMES[wt], M, e)
+    assert len(seen) == 6, seen
 
 
 @pytest.mark.parametrize("wt", G.ALL_TYPES, ids=lambda t: G.NAMES[t])

@@ -2,7 +2,7 @@
 array) against gqk_linear with a caller workspace, through the C ABI: bit-identical outputs on
 two calls in a row, the second with fewer rows, for a split-K GEMV plan, a slab-form GEMV plan (no
 workspace at all), the mid form (17..32 rows) in its slab and with its split-K exchange, a
-stream-K GEMM plan and a mixed-type layer; a plan whose workspace exceeds the array is refused
+split GEMM plan and a mixed-type layer; a plan whose workspace exceeds the array is refused
 with an error."""
 import ctypes
 
@@ -50,7 +50,7 @@ def test_noalloc_matches_linear_twice_then_smaller(dev):
         ("slab GEMV", [(G.Q6_K, 200)], 0, 8, (8, 3)),             # planned for 8 CUs: 7 slabs
         ("mid slab", [(G.Q4_K, 200)], 0, 8, (30, 17)),            # the mid form's slab, 7 slabs
         ("mid split-K", [(G.Q5_K, 900)], 4096, 0, (32, 20)),      # the mid form's exchange
-        ("stream-K GEMM", [(G.Q6_K, 1000)], 0, 0, (60, 20)),
+        ("split GEMM", [(G.Q6_K, 1000)], 0, 0, (60, 20)),
         ("mixed layer", [(G.IQ4_XS, 130), (G.Q5_K, 300), (G.Q8_0, 64)], 2048, 0, (5, 2)),
         ("mixed layer GEMM", [(G.IQ4_XS, 130), (G.Q5_K, 300), (G.Q8_0, 64)], 0, 0, (100, 33)),
     ]
