@@ -13,8 +13,8 @@
 namespace gqk {
 
 // Where a 256-weight record's bytes lie: RawSrc reads GGUF rows (any alignment), TileSrc a tile chunk in
-// LDS.  ld8<P>(j) / ld4 / ld2 / ld1: bytes j .. of plane P (j a multiple of the width; they never cross
-// a segment of the plane).
+// LDS.  ld<P, V>(j): the V at bytes j .. of plane P (j a multiple of its width; it never crosses a segment
+// of the plane); RawSrc::raw<V>(b): the V at byte b of the raw record.
 template <int T, int P>
 __device__ __forceinline__ int raw_of(int j) {   // raw byte of byte j of plane P (equal segments concatenated)
   constexpr gqk_plane pl = gqk_planes<T>::v.planes[P];

@@ -48,7 +48,7 @@ GLUON_TILE_TYPES = frozenset(ops.GGUF_TYPES)     # the types the loader holds in
 GLUON_DEQUANT_TYPES = frozenset()                # no run falls back to dequantize + a library GEMM
 GLUON_MAX_ROWS = 16                              # rows of the decode GEMV form
 GLUON_MAX_ROWS_GROUPED = 32                      # rows of the streaming forms (GEMV, then the mid form)
-GLUON_ARRIVAL_ROWS = 128                         # rows of the 128 x 128 GEMM tile form
+GLUON_ARRIVAL_ROWS = 128                         # rows up to which every GEMM plan has 128-row descriptor rows
 
 
 def _rec_bytes(weight_type: int) -> int:

@@ -44,10 +44,11 @@ GEMM_PLAN_M = (64, 128, 384, 512, 768, 769)
 # gluon_mul_mat_tiles_grouped dequantizes the tiles and runs the vendor bf16 GEMM above 128 rows
 # for the types its wide form loses on, gguf-plugin/gluon/interface.py:181-187): each shard is
 # decoded once by the tile dequant kernel and multiplied by torch's bf16 GEMM (hipBLASLt) in row
-# chunks.  Measured on the gate_up / down shards against the fused GEMM: at 8192 rows 12-44%
-# faster on gate_up for Q4_K, Q5_K, Q6_K, IQ4_XS and IQ3_S and, chunked, on `down`; at 4096 rows
-# 4-16%; at 2048 rows from even (Q4_K gate_up, the bench's line) to 12%, so the fused kernel keeps
-# those.  The chunk: DEQUANT_CHUNK_M rows, or DEQUANT_CHUNK_M_LONG_K for K above
+# chunks.  Measured against the fused GEMM (eight types, us fused -> regime): gate_up 34816 x 5120
+# at 2048 rows 637-700 -> 660-696, at 4096 1236-1371 -> 1284-1310, at 8192 2435-2748 -> 2166-2210;
+# down 5120 x 17408 319-351 -> 304-319, 618-681 -> 572-597, 1195-1337 -> 1129-1167; 7168 x 5120
+# 160-171 -> 120-126, 277-305 -> 218-224, 514-572 -> 417-435: right for the largest layers, late for
+# the smaller ones.  The chunk: DEQUANT_CHUNK_M rows, or DEQUANT_CHUNK_M_LONG_K for K above
 # DEQUANT_LONG_K - the vendor GEMM's 8192-row `down` (K = 17408) ran 2.5x its 4096-row time,
 # while gate_up (K = 5120) in two 4096-row chunks took 1.15x its one 8192-row call.
 DEQUANT_MIN_M = 4096
