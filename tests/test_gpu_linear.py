@@ -538,7 +538,7 @@ def test_baseline_config1_q8_0(dev):
     (17391, 5120, 2040, (8, 8, 1), True), (5101, 17408, 500, (8, 8, 1), True), (33000, 256, 401, (8, 8, 1), False),
 ], ids=str)
 @pytest.mark.parametrize("wt", [G.Q5_K, G.Q4_K, G.Q8_0], ids=lambda t: G.NAMES[t])
-def test_gemm_schedule(dev, n, K, M, geo, shared, wt):
+def test_gemm_stream_k_schedule(dev, n, K, M, geo, shared, wt):
     """The GEMM's schedules: one workgroup per tile and k-split (geometries below 256 tokens), split where
     the tiles are fewer than the CUs and K is long; the 256 x 256 form persistent, whole tiles dealt to the
     workgroups and the remainder tiles' super-blocks split over some of them (stream-K), remainder
